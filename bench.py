@@ -52,10 +52,9 @@ BYTES_PER_CELL = {
     "k_smag_scalar": 12,
     "k_copy": 8,
     # fused stage kernels (flow divergence computed inline, never stored)
-    "k_stage_scalars": 80,   # per scalar s, s0, sgs in + s_next out (x4: theta, qv, qc, qr); u, v, w in; theta_rho out
-    "k_mom_u": 20,           # u, v, w, sgs_u in; rhs_u out
-    "k_mom_v": 20,           # u, v, w, sgs_v in; rhs_v out
-    "k_mom_w": 28,           # u, v, w, theta, qv, sgs_w in; rhs_w out
+    # u, v, w, sgs_u in, rhs_u out (20); the same for v (20); u, v, w, theta, qv, sgs_w in, rhs_w
+    # out (28); u, v, w in, per scalar s, s0, sgs in and s_next out (x4), theta_rho out (80)
+    "k_stage": 148,
     "k_smag_fused": 56,      # u, v, w, theta, qv, qc, qr in; sgs_u, sgs_v, sgs_w and 4 scalar tendencies out
 }
 

@@ -175,34 +175,21 @@ void rk3_forward_tape(const Dims& d, const O& o, const B& b, float* const* X0, c
     }
     // the fused stage kernels of the forward step where they apply (same trajectory as
     // lex_rk3_step impl 0), else one kernel per reference routine
-    const int nzl = 64 * ((d.nz + 63) / 64);
-    const bool fused = nzl * kFTY <= 1024 && nsc >= 2 && nsc <= 6;
+    const bool fused = stage_ok(d, nsc);
     if (fused) {
-      dim3 fb(nzl, kFTY, 1), fg((d.nx + kFTX - 1) / kFTX, (d.ny + kFTY - 1) / kFTY, 1);
+      StageArgs a;
+      a.rc = rc; a.th0c = b.theta0; a.qv0c = b.qv0;
+      a.u = src[1]; a.v = src[2]; a.w = src[3]; a.th = src[0]; a.qv = src[5];
+      a.su = turb ? su : nullptr; a.sv = turb ? sv : nullptr; a.sw = turb ? sw : nullptr;
+      a.tau_x = a.tau_y = nullptr;
       // the taped forward covers cor_opt 0 (its reverse has no Coriolis term; the entry
       // points reject cor != 0)
-      const CorOpt nocor{0, 0.0f, 0.0f, 0.0f};
-      hipLaunchKernelGGL(k_mom_u, fg, fb, mom_uv_lds(d), st, d, rc, src[1], src[2], src[3],
-                         turb ? (const float*)su : nullptr, (const float*)nullptr, nocor, ru);
-      hipLaunchKernelGGL(k_mom_v, fg, fb, mom_uv_lds(d), st, d, rc, src[1], src[2], src[3],
-                         turb ? (const float*)sv : nullptr, (const float*)nullptr, nocor, rv);
-      hipLaunchKernelGGL(k_mom_w, fg, fb, mom_w_lds(d), st, d, rc, b.theta0, b.qv0, src[1], src[2], src[3], src[0],
-                         src[5], turb ? (const float*)sw : nullptr, rw);
-      ScalarSet S;
-      S.heat = nullptr;
-      S.n = nsc;
-      for (int q = 0; q < nsc; ++q) {
-        int fi = (q == 0) ? 0 : (q == 1 ? 5 : 6 + (q - 2));
-        S.s0[q] = X0[fi];
-        S.s[q] = src[fi];
-        S.sgs[q] = turb ? ss[q] : nullptr;
-        S.out[q] = dst[fi];
-        S.weps[q] = (q == 0) ? 1.0e-17f : 1.0e-18f;
-      }
-      size_t lds = stage_scalars_lds(d);
-      float dts_f = (float)dt_s;
-      hipLaunchKernelGGL(k_stage_scalars, dim3(nsc, fg.x, fg.y), fb, lds, st, d, rc, src[1], src[2], src[3], S, tr,
-                         dts_f);
+      a.cor = CorOpt{0, 0.0f, 0.0f, 0.0f};
+      a.ru = ru; a.rv = rv; a.rw = rw;
+      stage_scalar_set(a.S, o.n_passive, X0, src, turb ? ss : nullptr, dst);
+      a.trho = tr;
+      a.dt = (float)dt_s;
+      launch_stage(d, a, st);
     } else {
       hipLaunchKernelGGL(k_div_rho, cx.G(d.nz + 2, d.ny + 6, d.nx + 6), cx.bk, 0, st, d, rc, src[1], src[2], src[3],
                          fd);

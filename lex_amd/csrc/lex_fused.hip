@@ -1,25 +1,30 @@
 // Fused stage kernels for the device WS-RK3 driver.
 //
-// k_stage_scalars: the scalars' WENO advection + Euler update + frozen-SGS add-in of
-// one stage (update_theta_euler / update_qv_euler, one_step_integration.py:450-465,
-// :158-162), plus the flow divergence (advection.py:200-226) and theta_rho
-// (one_step_integration.py:135) inline, in one launch (one scalar per workgroup).
+// k_stage: everything of one stage that reads only its input state, in one launch: the
+// momentum right-hand sides (mom_u/v/w_tile) and, one scalar per workgroup (scalar_tile),
+// the scalars' WENO advection + Euler update + frozen-SGS add-in
+// (update_theta_euler / update_qv_euler, one_step_integration.py:450-465, :158-162), with
+// the flow divergence (advection.py:200-226) and theta_rho (one_step_integration.py:135)
+// inline.
 //
 // Work decomposition (each face flux computed once):
-//   block  = full z column (64*ceil(nz/64) lanes) x TY rows of y of one scalar; marches
-//            TX cells in x
+//   block  = full z column (64*ceil(nz/64) lanes) x TY rows of y of one piece; marches
+//            ax cells in x (stage_ax)
 //   x-face : from a 6-value register window along x; the lower face is the previous
 //            step's upper face
 //   y-face : each row computes its lower face from an LDS plane (rows j0-3..j0+TY+2);
 //            the last row also computes the tile's upper face
 //   z-face : each lane its lower face from the LDS column; the lid face is zero
 #pragma once
+#include <math.h>
+#include <algorithm>
 #include "lex_common.hpp"
+#include "lex_prof.hpp"
 
 namespace lex {
 
 constexpr int kFTY = 4;    // rows of y per block
-constexpr int kFTX = 16;   // cells marched in x per block
+constexpr int kFTX = 16;   // cells marched in x per block, at most (k_stage)
 constexpr int kMaxScalars = 8;
 constexpr int kSlots = 3;  // ceil((kFTY + 6) * L / (64 * ceil(nz / 64) * kFTY)) <= 3 for L <= nz + 3
 
@@ -98,6 +103,11 @@ __device__ __forceinline__ BottomFlux bottom_fluxes(const ScalarSet& S, bool sur
   return b;
 }
 
+// What one workgroup of the fused stage works on: rows j0..j0+kFTY-1, cells i0..iend-1.
+struct StageTile {
+  int i0, iend, j0;
+};
+
 // Flow divergence div(rho0 u) of a cell (get_divergence, advection.py:200-226) for a
 // horizontally uniform rho column, from the cell's face velocities already in registers:
 // r = rho at the cell, r8lo / r8hi at its lower / upper w level (zero at the ghost levels).
@@ -113,22 +123,21 @@ __device__ __forceinline__ float fd_ops(const Dims& d, float r, float r8lo, floa
 // from the previous step.
 
 // ---------------------------------------------------------------------------------
-// k_mom_u: rhs_u = advection_u + sgs_u at u faces 0..nx-1 (face nx is the periodic
+// mom_u_tile: rhs_u = advection_u + sgs_u at u faces 0..nx-1 (face nx is the periodic
 // duplicate of face 0 and is written from it).  advection.py:37-74, :561-771.
 // ---------------------------------------------------------------------------------
-__global__ void __launch_bounds__(1024) k_mom_u(Dims d, const float* __restrict__ rc, const float* __restrict__ u,
-                                                 const float* __restrict__ v, const float* __restrict__ w,
-                                                 const float* __restrict__ sgs, const float* __restrict__ tau_x,
-                                                 CorOpt cor, float* __restrict__ ru) {
-  extern __shared__ float lds[];
+__device__ __forceinline__ void mom_u_tile(const Dims& d, const StageTile& tb, float* lds,
+                                           const float* __restrict__ rc, const float* __restrict__ u,
+                                           const float* __restrict__ v, const float* __restrict__ w,
+                                           const float* __restrict__ sgs, const float* __restrict__ tau_x,
+                                           const CorOpt& cor, float* __restrict__ ru) {
   const float weps = 1.0e-16f;
   const int nzl = blockDim.x, tz = threadIdx.x, ty = threadIdx.y, nt = nzl * kFTY, tid = ty * nzl + tz;
   const int Lz = d.nz + 2;
   float* P = lds;
   float* FY = P + (kFTY + 6) * Lz;
   float* FZ = FY + (kFTY + 1) * nzl;
-  const TileId tb = xcd_tile();
-  const int j0 = tb.y * kFTY, i0 = tb.x * kFTX;
+  const int j0 = tb.j0, i0 = tb.i0;
   const int k = lane_level(tz, nzl, d.nz), j = j0 + ty;
   const bool act = (k < d.nz) && (j < d.ny);
   const int K = k + 1;
@@ -139,7 +148,7 @@ __global__ void __launch_bounds__(1024) k_mom_u(Dims d, const float* __restrict_
   const float r8lo = (Kc <= 0 || Kc >= d.nz + 2) ? 0.0f : 0.5f * (rc[Kc - 1] + rc[Kc]);
   const float r8hi = (Kc + 1 >= d.nz + 2) ? 0.0f : 0.5f * (rc[Kc] + rc[Kc + 1]);
   const float r8w = 0.5f * (rc[Kc - 1] + rc[Kc]);   // rho at the w level below (z mass flux)
-  const int iend = min(i0 + kFTX, d.nx);
+  const int iend = tb.iend;
   const PlaneSlots psl = plane_slots(tid, nt, Lz, j0, d.ny + 5, (int)d.syc());
   const uint32_t usx = (uint32_t)d.sxu(), usy = (uint32_t)d.syc();
   const uint32_t usxv = (uint32_t)d.sxv(), usxw = (uint32_t)d.sxw(), usyw = (uint32_t)d.syw();
@@ -233,22 +242,21 @@ __global__ void __launch_bounds__(1024) k_mom_u(Dims d, const float* __restrict_
 }
 
 // ---------------------------------------------------------------------------------
-// k_mom_v: rhs_v = advection_v + sgs_v at v faces 0..ny-1 (face ny written from 0).
+// mom_v_tile: rhs_v = advection_v + sgs_v at v faces 0..ny-1 (face ny written from 0).
 // advection.py:77-114, :816-1025.
 // ---------------------------------------------------------------------------------
-__global__ void __launch_bounds__(1024) k_mom_v(Dims d, const float* __restrict__ rc, const float* __restrict__ u,
-                                                 const float* __restrict__ v, const float* __restrict__ w,
-                                                 const float* __restrict__ sgs, const float* __restrict__ tau_y,
-                                                 CorOpt cor, float* __restrict__ rv) {
-  extern __shared__ float lds[];
+__device__ __forceinline__ void mom_v_tile(const Dims& d, const StageTile& tb, float* lds,
+                                           const float* __restrict__ rc, const float* __restrict__ u,
+                                           const float* __restrict__ v, const float* __restrict__ w,
+                                           const float* __restrict__ sgs, const float* __restrict__ tau_y,
+                                           const CorOpt& cor, float* __restrict__ rv) {
   const float weps = 1.0e-16f;
   const int nzl = blockDim.x, tz = threadIdx.x, ty = threadIdx.y, nt = nzl * kFTY, tid = ty * nzl + tz;
   const int Lz = d.nz + 2;
   float* P = lds;
   float* FY = P + (kFTY + 6) * Lz;
   float* FZ = FY + (kFTY + 1) * nzl;
-  const TileId tb = xcd_tile();
-  const int j0 = tb.y * kFTY, i0 = tb.x * kFTX;
+  const int j0 = tb.j0, i0 = tb.i0;
   const int k = lane_level(tz, nzl, d.nz), j = j0 + ty;
   const bool act = (k < d.nz) && (j < d.ny);
   const int K = k + 1;
@@ -259,7 +267,7 @@ __global__ void __launch_bounds__(1024) k_mom_v(Dims d, const float* __restrict_
   const float r8lo = (Kc <= 0 || Kc >= d.nz + 2) ? 0.0f : 0.5f * (rc[Kc - 1] + rc[Kc]);
   const float r8hi = (Kc + 1 >= d.nz + 2) ? 0.0f : 0.5f * (rc[Kc] + rc[Kc + 1]);
   const float r8w = 0.5f * (rc[Kc - 1] + rc[Kc]);
-  const int iend = min(i0 + kFTX, d.nx);
+  const int iend = tb.iend;
   const PlaneSlots psl = plane_slots(tid, nt, Lz, j0, d.ny + 6, (int)d.syc());
   const uint32_t usx = (uint32_t)d.sxv(), usy = (uint32_t)d.syc();
   const uint32_t usxu = (uint32_t)d.sxu(), usxw = (uint32_t)d.sxw(), usyw = (uint32_t)d.syw();
@@ -350,19 +358,17 @@ __global__ void __launch_bounds__(1024) k_mom_v(Dims d, const float* __restrict_
 }
 
 // ---------------------------------------------------------------------------------
-// k_mom_w: rhs_w = advection_w + b8w + sgs_w at w levels 0..nz (advection.py:117-149,
+// mom_w_tile: rhs_w = advection_w + b8w + sgs_w at w levels 0..nz (advection.py:117-149,
 // :1070-1281; pressure_equations.py:162-172).  Lane l owns level l and computes the
 // vertical flux at scalar level l+1 (its upper face); the lid level is written by the
 // top lane.
 // ---------------------------------------------------------------------------------
-// 80 VGPRs at most: six waves per SIMD, three 512-thread workgroups per CU (at 93 the
-// compiler's choice, two)
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6))) k_mom_w(Dims d, const float* __restrict__ rc, const float* __restrict__ th0c,
-                                                 const float* __restrict__ qv0c, const float* __restrict__ u,
-                                                 const float* __restrict__ v, const float* __restrict__ w,
-                                                 const float* __restrict__ th, const float* __restrict__ qv,
-                                                 const float* __restrict__ sgs, float* __restrict__ rw) {
-  extern __shared__ float lds[];
+__device__ __forceinline__ void mom_w_tile(const Dims& d, const StageTile& tb, float* lds,
+                                           const float* __restrict__ rc, const float* __restrict__ th0c,
+                                           const float* __restrict__ qv0c, const float* __restrict__ u,
+                                           const float* __restrict__ v, const float* __restrict__ w,
+                                           const float* __restrict__ th, const float* __restrict__ qv,
+                                           const float* __restrict__ sgs, float* __restrict__ rw) {
   const float weps = 1.0e-16f;
   const int nzl = blockDim.x, tz = threadIdx.x, ty = threadIdx.y, nt = nzl * kFTY, tid = ty * nzl + tz;
   const int Lw = d.nz + 3;
@@ -371,8 +377,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6))) 
   float* FZ = FY + (kFTY + 1) * nzl;                // kFTY x nzl: flux at scalar level l+1
   float* FD = FZ + kFTY * nzl;                      // kFTY x nzl: flow divergence at cell l
   float* BB = FD + kFTY * nzl;                      // kFTY x nzl: buoyancy at cell l
-  const TileId tb = xcd_tile();
-  const int j0 = tb.y * kFTY, i0 = tb.x * kFTX;
+  const int j0 = tb.j0, i0 = tb.i0;
   const int l = lane_level(tz, nzl, d.nz), j = j0 + ty;
   const bool row_ok = j < d.ny;
   const bool lane_ok = l < d.nz;                   // owns level l and cell l
@@ -386,7 +391,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6))) 
   const float rK = rc[Kc];
   const float r8lo = (Kc <= 0 || Kc >= d.nz + 2) ? 0.0f : 0.5f * (rc[Kc - 1] + rc[Kc]);
   const float r8hi = (Kc + 1 >= d.nz + 2) ? 0.0f : 0.5f * (rc[Kc] + rc[Kc + 1]);
-  const int iend = min(i0 + kFTX, d.nx);
+  const int iend = tb.iend;
   const PlaneSlots psl = plane_slots(tid, nt, Lw, j0, d.ny + 5, (int)d.syw());
   const uint32_t usx = (uint32_t)d.sxw(), usyw = (uint32_t)d.syw();
   const uint32_t usxu = (uint32_t)d.sxu(), usy = (uint32_t)d.syc(), usxv = (uint32_t)d.sxv();
@@ -489,15 +494,6 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6))) 
   }
 }
 
-inline size_t mom_uv_lds(const Dims& d) {
-  int nzl = 64 * ((d.nz + 63) / 64);
-  return sizeof(float) * ((size_t)(kFTY + 6) * (d.nz + 2) + (size_t)(2 * kFTY + 1) * nzl);
-}
-inline size_t mom_w_lds(const Dims& d) {
-  int nzl = 64 * ((d.nz + 63) / 64);
-  return sizeof(float) * ((size_t)(kFTY + 6) * (d.nz + 3) + (size_t)(4 * kFTY + 1) * nzl);
-}
-
 // The entry of a per-scalar array of ScalarSet for a wave-uniform scalar index q
 // (a select chain on scalar registers, not an indexed copy of the argument struct).
 template <class T>
@@ -509,20 +505,17 @@ __device__ __forceinline__ T pick_q(const T (&a)[kMaxScalars], int q) {
 }
 
 // ---------------------------------------------------------------------------------
-// k_stage_scalars: one scalar's WENO advection + Euler update + frozen-SGS add-in per
-// workgroup.  The grid's fastest dimension is the scalar, so the workgroups of the S.n
-// scalars of one tile are consecutive, run on the same XCD and share the tile's u, v, w
-// lines in its L2; each recomputes the tile's mass fluxes and flow divergence.  Holding
+// scalar_tile: one scalar's WENO advection + Euler update + frozen-SGS add-in.  Each
+// scalar's workgroup recomputes the tile's mass fluxes and flow divergence.  Holding
 // one scalar's x window (not all S.n) keeps the kernel at 80 VGPRs: three workgroups per
 // CU, whose barriers and loads overlap (the all-scalars-per-workgroup form needed 119 and
 // ran one fewer, 12 % slower).  theta_rho is written by the workgroups of scalar 0
 // (theta), which read qv at their cells.
 // ---------------------------------------------------------------------------------
-__global__ void __launch_bounds__(1024) k_stage_scalars(Dims d, const float* __restrict__ rc,
-                                                        const float* __restrict__ u, const float* __restrict__ v,
-                                                        const float* __restrict__ w, ScalarSet S,
-                                                        float* __restrict__ trho, float dt) {
-  extern __shared__ float lds[];
+__device__ __forceinline__ void scalar_tile(const Dims& d, const StageTile& tb, float* lds, int q,
+                                            const float* __restrict__ rc, const float* __restrict__ u,
+                                            const float* __restrict__ v, const float* __restrict__ w,
+                                            const ScalarSet& S, float* __restrict__ trho, float dt) {
   const int nzl = blockDim.x;
   const int tz = threadIdx.x, ty = threadIdx.y;
   const int nt = nzl * kFTY;
@@ -532,10 +525,7 @@ __global__ void __launch_bounds__(1024) k_stage_scalars(Dims d, const float* __r
   float* FY = P + (kFTY + 6) * Lz;
   float* FZ = FY + (kFTY + 1) * nzl;
 
-  const TileId tb = xcd_tile();
-  const int q = tb.x;
-  const int i0 = tb.y * kFTX;
-  const int j0 = tb.z * kFTY;
+  const int i0 = tb.i0, j0 = tb.j0;
   const float* __restrict__ s = pick_q(S.s, q);
   const float* __restrict__ s0 = pick_q(S.s0, q);
   const float* __restrict__ sgs = pick_q(S.sgs, q);
@@ -566,7 +556,7 @@ __global__ void __launch_bounds__(1024) k_stage_scalars(Dims d, const float* __r
   uint32_t op = (uint32_t)(i0 + 3) * usx;
   float win[6];
   float fxlo;
-  const int iend = min(i0 + kFTX, d.nx);
+  const int iend = tb.iend;
   {
     const float mlo = r * ld32(u, oc);
     const bool pos = upwind_pos(mlo);
@@ -639,16 +629,97 @@ __global__ void __launch_bounds__(1024) k_stage_scalars(Dims d, const float* __r
   }
 }
 
-inline size_t stage_scalars_lds(const Dims& d) {
-  int nzl = 64 * ((d.nz + 63) / 64);
-  return sizeof(float) * ((size_t)(kFTY + 6) * (d.nz + 2) + (size_t)(kFTY + 1) * nzl + (size_t)kFTY * nzl);
+// ---------------------------------------------------------------------------------
+// k_stage: everything of a stage that reads only its input state, in one launch.  The
+// grid's fastest dimension is the piece (rhs_u, rhs_v, rhs_w, then one per scalar), so the
+// workgroups of one tile are consecutive, run on one XCD and share the tile's u, v, w
+// lines in its L2.  One launch instead of four (u, v, w, scalars) keeps the chip full where
+// a piece alone would leave it idle, and has one last round instead of four: VALU issue
+// bounds it on large grids (256x256x128, four scalars: 595 us in four launches, 534 in
+// one), the length of a workgroup's march on small ones (40x40x40, two scalars: 132 us per
+// stage in four launches of 16-cell marches, 13 in one of two-cell marches).
+// ---------------------------------------------------------------------------------
+struct StageArgs {
+  const float *rc, *th0c, *qv0c;      // base columns
+  const float *u, *v, *w, *th, *qv;   // stage state
+  const float *su, *sv, *sw;          // frozen SGS tendencies or null
+  const float *tau_x, *tau_y;         // surface stresses or null
+  CorOpt cor;
+  float *ru, *rv, *rw;                // momentum right-hand sides
+  ScalarSet S;
+  float* trho;
+  float dt;
+};
+
+// 80 VGPRs at most: six waves per SIMD, three 512-thread workgroups per CU (at 93, the
+// compiler's choice for the w piece, two)
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6))) k_stage(Dims d, StageArgs a, int ax) {
+  extern __shared__ float lds[];
+  const TileId t = xcd_tile();
+  StageTile tb;
+  tb.i0 = t.y * ax;
+  tb.iend = min(tb.i0 + ax, d.nx);
+  tb.j0 = t.z * kFTY;
+  if (t.x == 0)
+    mom_u_tile(d, tb, lds, a.rc, a.u, a.v, a.w, a.su, a.tau_x, a.cor, a.ru);
+  else if (t.x == 1)
+    mom_v_tile(d, tb, lds, a.rc, a.u, a.v, a.w, a.sv, a.tau_y, a.cor, a.rv);
+  else if (t.x == 2)
+    mom_w_tile(d, tb, lds, a.rc, a.th0c, a.qv0c, a.u, a.v, a.w, a.th, a.qv, a.sw, a.rw);
+  else
+    scalar_tile(d, tb, lds, t.x - 3, a.rc, a.u, a.v, a.w, a.S, a.trho, a.dt);
+}
+
+// The scalars of a stage: theta, qv and n_passive more, from the padded fields x0 (the
+// step's input), x (the stage's) and out, in state order; sgs: tendencies or null.
+inline void stage_scalar_set(ScalarSet& S, int n_passive, float* const* x0, float* const* x, float* const* sgs,
+                             float* const* out) {
+  S.n = 2 + n_passive;
+  for (int q = 0; q < S.n; ++q) {
+    const int fi = (q == 0) ? 0 : (q == 1 ? 5 : 6 + (q - 2));
+    S.s0[q] = x0[fi];
+    S.s[q] = x[fi];
+    S.sgs[q] = sgs ? sgs[q] : nullptr;
+    S.out[q] = out[fi];
+    S.weps[q] = (q == 0) ? 1.0e-17f : 1.0e-18f;
+  }
+}
+
+inline bool stage_ok(const Dims& d, int nsc) { return 64 * ((d.nz + 63) / 64) * kFTY <= 1024 && nsc >= 2 && nsc <= 6; }
+
+inline size_t stage_lds(const Dims& d) {   // the w piece's, the largest
+  const int nzl = 64 * ((d.nz + 63) / 64);
+  return sizeof(float) * ((size_t)(kFTY + 6) * (d.nz + 3) + (size_t)(4 * kFTY + 1) * nzl);
+}
+
+// Cells marched along x per workgroup.  A workgroup of ax cells costs about ax + 1 x-steps
+// (the first face and the window loads are the extra one), so with N = pieces x row tiles x
+// nx columns on `slots` resident workgroups a launch takes N (ax + 1) / (ax slots) steps
+// plus, on average, half a workgroup of ax + 1 in a last round that is not full: least at
+// ax = sqrt(2 N / slots).  Measured steps in us, ax = 1, 4, 8, 16, 32: 40x40x40 (ax 2 here)
+// 165, 178, 201, 252, 357; 96x96x48 with the closure (4) 420, 397, 405, 441, 547;
+// 181x147x70 with three scalars (10) 1546, 1277, 1247, 1274, 1340; 256x256x128 with four
+// scalars (16) 4034, 3190, 3085, 3059, 3104.  Within the bound the tiles are made even.
+inline int stage_ax(const Dims& d, int pieces) {
+  const int threads = 64 * ((d.nz + 63) / 64) * kFTY;
+  const int slots = 256 * (24 * 64 / threads);   // 24 waves per CU at 80 VGPRs
+  const double n = (double)pieces * ((d.ny + kFTY - 1) / kFTY) * d.nx;
+  const int ax = std::min(kFTX, std::max(1, (int)lround(sqrt(2.0 * n / slots))));
+  const int tiles = (d.nx + ax - 1) / ax;
+  return (d.nx + tiles - 1) / tiles;
+}
+
+inline void launch_stage(const Dims& d, const StageArgs& a, hipStream_t st) {
+  const int pieces = 3 + a.S.n, ax = stage_ax(d, pieces);
+  LEX_LAUNCH(KID_STAGE, k_stage, dim3(pieces, (d.nx + ax - 1) / ax, (d.ny + kFTY - 1) / kFTY),
+             dim3(64 * ((d.nz + 63) / 64), kFTY, 1), stage_lds(d), st, d, a, ax);
 }
 
 // ---------------------------------------------------------------------------------
-// k_stage_scalars_db: the same arithmetic as k_stage_scalars, all scalars per workgroup:
+// k_stage_scalars_db: the same arithmetic as scalar_tile, all scalars per workgroup:
 // the planes of all NS scalars at x = I+1 are fetched into registers at the start of
 // step I and written to the second of two LDS plane buffers after the step's face
-// fluxes, so one x-step takes two barriers for all scalars (k_stage_scalars: two per
+// fluxes, so one x-step takes two barriers for all scalars (scalar_tile: two per
 // scalar) and the global loads overlap the WENO arithmetic.
 // LDS: 2 x NS planes + NS x (2 kFTY + 1) face rows.
 // ---------------------------------------------------------------------------------

@@ -428,60 +428,47 @@ int rk3_step(const Dims& d, const O& o, const B& b, float* const* state, char* w
       }
     }
     const int nsc = 2 + o.n_passive;
-    const bool fused_ok = (64 * ((d.nz + 63) / 64)) * kFTY <= 1024 && nsc >= 2 && nsc <= 6;
-    // impl 0: fused stage kernels; impl 2: the same with the double-buffered scalar kernel;
-    // impl 1: one kernel per reference routine
+    const bool fused_ok = stage_ok(d, nsc);
+    // impl 0: the fused stage kernel; impl 2: the same for the momentum, with the
+    // double-buffered scalar kernel; impl 1: one kernel per reference routine
     const bool fused = (o.impl == 0 || o.impl == 2);
     if (fused && !fused_ok) return -4;  // the caller falls back to impl 1
     if (o.impl == 2 && (stage_scalars_db_lds(d, nsc) > 65536 || 64 * ((d.nz + 63) / 64) * kFTY > 512)) return -4;
     if (fused) {
-      const int nzl = 64 * ((d.nz + 63) / 64);
-      dim3 fb(nzl, kFTY, 1), fg((d.nx + kFTX - 1) / kFTX, (d.ny + kFTY - 1) / kFTY, 1);
-      LEX_LAUNCH(KID_STAGE_MOMENTUM, k_mom_u, fg, fb, mom_uv_lds(d), st, d, rc, src[1], src[2], src[3],
-                 turb ? (const float*)su : nullptr, tau_x, cor, ru);
-      LEX_LAUNCH(KID_MOM_V, k_mom_v, fg, fb, mom_uv_lds(d), st, d, rc, src[1], src[2], src[3],
-                 turb ? (const float*)sv : nullptr, tau_y, cor, rv);
-      LEX_LAUNCH(KID_MOM_W, k_mom_w, fg, fb, mom_w_lds(d), st, d, rc, b.theta0, b.qv0, src[1], src[2], src[3],
-                 src[0], src[5], turb ? (const float*)sw : nullptr, rw);
+      StageArgs a;
+      a.rc = rc; a.th0c = b.theta0; a.qv0c = b.qv0;
+      a.u = src[1]; a.v = src[2]; a.w = src[3]; a.th = src[0]; a.qv = src[5];
+      a.su = turb ? su : nullptr; a.sv = turb ? sv : nullptr; a.sw = turb ? sw : nullptr;
+      a.tau_x = tau_x; a.tau_y = tau_y;
+      a.cor = cor;
+      a.ru = ru; a.rv = rv; a.rw = rw;
+      stage_scalar_set(a.S, o.n_passive, X0, src, turb ? ss : nullptr, dst);
+      a.S.heat = heat;
+      a.S.sfc[0] = sen_cp;
+      a.S.sfc[1] = evap;
+      a.trho = tr;
+      a.dt = (float)dt_s;
+      if (o.impl == 2) {
+        const ScalarSet S = a.S;
+        a.S.n = 0;
+        launch_stage(d, a, st);
+        const dim3 fb(64 * ((d.nz + 63) / 64), kFTY, 1), fg((d.nx + kFTX - 1) / kFTX, (d.ny + kFTY - 1) / kFTY, 1);
+        const size_t ldb = stage_scalars_db_lds(d, nsc);
+        switch (nsc) {
+          case 2: LEX_LAUNCH(KID_STAGE_SCALARS, k_stage_scalars_db<2>, fg, fb, ldb, st, d, rc, src[1], src[2], src[3], S, tr, a.dt); break;
+          case 3: LEX_LAUNCH(KID_STAGE_SCALARS, k_stage_scalars_db<3>, fg, fb, ldb, st, d, rc, src[1], src[2], src[3], S, tr, a.dt); break;
+          case 4: LEX_LAUNCH(KID_STAGE_SCALARS, k_stage_scalars_db<4>, fg, fb, ldb, st, d, rc, src[1], src[2], src[3], S, tr, a.dt); break;
+          default: return -4;
+        }
+      } else {
+        launch_stage(d, a, st);
+      }
     } else {
       LEX_LAUNCH(KID_DIV_RHO, k_div_rho, G(d.nz + 2, d.ny + 6, d.nx + 6), bk, 0, st, d, rc, src[1], src[2], src[3], fd);
       LEX_LAUNCH(KID_RHS_UV, k_rhs_uv, G(d.nz, d.ny + 1, d.nx + 1), bk, 0, st, d, rc, src[1], src[2], src[3], fd,
                  turb ? su : nullptr, turb ? sv : nullptr, tau_x, tau_y, cor, ru, rv);
       LEX_LAUNCH(KID_RHS_W, k_rhs_w, G(d.nz + 1, d.ny, d.nx), bk, 0, st, d, rc, b.theta0, b.qv0, src[1], src[2], src[3],
                  src[0], src[5], fd, turb ? sw : nullptr, rw);
-    }
-    if (fused) {
-      // all scalars of the stage + theta_rho in one launch (k_stage_scalars)
-      ScalarSet S;
-      S.n = nsc;
-      for (int q = 0; q < nsc; ++q) {
-        int fi = (q == 0) ? 0 : (q == 1 ? 5 : 6 + (q - 2));
-        S.s0[q] = X0[fi];
-        S.s[q] = src[fi];
-        S.sgs[q] = turb ? ss[q] : nullptr;
-        S.out[q] = dst[fi];
-        S.weps[q] = (q == 0) ? 1.0e-17f : 1.0e-18f;
-      }
-      S.heat = heat;
-      S.sfc[0] = sen_cp;
-      S.sfc[1] = evap;
-      const int nzl = 64 * ((d.nz + 63) / 64);
-      dim3 fb(nzl, kFTY, 1), fg((d.nx + kFTX - 1) / kFTX, (d.ny + kFTY - 1) / kFTY, 1);
-      size_t lds = stage_scalars_lds(d);
-      float dts_f = (float)dt_s;
-      if (o.impl == 2) {
-        size_t ldb = stage_scalars_db_lds(d, nsc);
-        switch (nsc) {
-          case 2: LEX_LAUNCH(KID_STAGE_SCALARS, k_stage_scalars_db<2>, fg, fb, ldb, st, d, rc, src[1], src[2], src[3], S, tr, dts_f); break;
-          case 3: LEX_LAUNCH(KID_STAGE_SCALARS, k_stage_scalars_db<3>, fg, fb, ldb, st, d, rc, src[1], src[2], src[3], S, tr, dts_f); break;
-          case 4: LEX_LAUNCH(KID_STAGE_SCALARS, k_stage_scalars_db<4>, fg, fb, ldb, st, d, rc, src[1], src[2], src[3], S, tr, dts_f); break;
-          default: return -4;
-        }
-      } else {
-        dim3 g1(nsc, (d.nx + kFTX - 1) / kFTX, (d.ny + kFTY - 1) / kFTY);   // scalar fastest
-        LEX_LAUNCH(KID_STAGE_SCALARS, k_stage_scalars, g1, fb, lds, st, d, rc, src[1], src[2], src[3], S, tr, dts_f);
-      }
-    } else {
       long n = (long)L.nc;
       LEX_LAUNCH(KID_THETA_RHO, k_theta_rho, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, src[0], src[5], tr);
     }
