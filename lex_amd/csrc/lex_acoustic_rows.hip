@@ -1,0 +1,365 @@
+// S1: one forward-backward acoustic substep (one_step_integration.py:528-553), V levels per
+// lane, marched along x.
+//
+// A wave owns one row of y and 64 V levels, lane l the levels V l .. V l + V - 1, and marches
+// `ax` cells along x with no barrier and no LDS: the x neighbours and the x face below are
+// carried in registers, the z neighbours are the lane's other level or the adjacent lane's
+// (a wave shift in the vector pipe), and the x and z faces are evaluated once.  Two levels
+// per lane halve the vector-memory instructions, which kept the address unit of the
+// cell-per-thread form 77 % busy (29 loads per cell; here 10 for one level, 20 of 8 bytes
+// for two).
+//
+// The arithmetic is acoustic_cell's operation by operation (contraction off, fmaf where it
+// has one), so the result is bit for bit that of k_acoustic2 and of a cell-per-thread
+// evaluation.
+#pragma once
+#include <algorithm>
+#include "lex_ops.hip"
+#include "lex_prof.hpp"
+
+namespace lex {
+
+// Two floats at a 4-byte aligned address in one access.
+struct __attribute__((packed, aligned(4))) Pair32 {
+  float x, y;
+};
+
+template <int V>
+__device__ __forceinline__ void ld_levels(const float* __restrict__ row, uint32_t e, float (&o)[V]) {
+  if constexpr (V == 1) {
+    o[0] = ld32(row, e);
+  } else {
+    const Pair32 t = *reinterpret_cast<const Pair32*>(reinterpret_cast<const char*>(row) + (size_t)(e * 4u));
+    o[0] = t.x;
+    o[1] = t.y;
+  }
+}
+// The same from an unpadded row: the lane whose second level would lie past the row (odd nz)
+// reads one level lower (e already is) and takes the upper value as its first.
+template <int V>
+__device__ __forceinline__ void ld_levels_in(const float* __restrict__ row, uint32_t e, bool past, float (&o)[V]) {
+  ld_levels<V>(row, e, o);
+  if constexpr (V == 2) o[0] = past ? o[1] : o[0];
+}
+
+// The value of the lane below / above (DPP wave shift by one); lane 0 / 63 get 0.
+__device__ __forceinline__ float lane_below(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_above(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130, 0xf, 0xf, false));
+}
+
+// Where a lane's levels go in a padded column: n of its V levels exist, the first / last of
+// the column also fill the z ghosts.
+struct LevelSlots {
+  int n;
+  bool first, last;
+};
+
+// Store the lane's levels at element e (its first level) of a padded field.
+template <int V>
+__device__ __forceinline__ void st_levels(float* __restrict__ f, uint32_t e, const LevelSlots& s, const float (&val)[V]) {
+  if (V == 2 && s.n == 2) {
+    Pair32 t;
+    t.x = val[0];
+    t.y = val[V - 1];
+    *reinterpret_cast<Pair32*>(reinterpret_cast<char*>(f) + (size_t)(e * 4u)) = t;
+  } else if (s.n >= 1) {
+    st32(f, e, val[0]);
+  }
+}
+// The z ghosts of a column: copies of its first and last level.
+template <int V>
+__device__ __forceinline__ void st_ghosts(float* __restrict__ f, uint32_t e, const LevelSlots& s, const float (&val)[V]) {
+  if (s.first) st32(f, e - 1u, val[0]);
+  if (s.last) st32(f, e + (uint32_t)s.n, (V == 2 && s.n == 2) ? val[V - 1] : val[0]);
+}
+// w: the lid level and its ghost above the last cell are zero.
+template <int V>
+__device__ __forceinline__ void st_ghosts_w(float* __restrict__ f, uint32_t e, const LevelSlots& s, const float (&val)[V]) {
+  if (s.first) st32(f, e - 1u, val[0]);
+  if (s.last) {
+    st32(f, e + (uint32_t)s.n, 0.0f);
+    st32(f, e + (uint32_t)s.n + 1u, 0.0f);
+  }
+}
+
+// Periodic images of index i on an axis of n cells (face: of n + 1 faces, whose ghosts skip
+// the duplicate), as a mask: bit 0 the point itself, 1 its image one period up, 2 down.
+__device__ __forceinline__ int image_mask(int i, int n, bool face) {
+  if (face) return 1 | ((i >= 1 && i <= 3) ? 2 : 0) | ((i >= n - 3 && i <= n - 1) ? 4 : 0);
+  return 1 | (i < 3 ? 2 : 0) | (i >= n - 3 ? 4 : 0);
+}
+
+// Store a column of point (i, j) and its periodic images; i, j uniform over the wave, sx and
+// sy the field's strides, e the lane's first level within a column.
+template <int V, bool ONW>
+__device__ __forceinline__ void st_images(float* __restrict__ f, int sx, int sy, int i, int nx, bool fx, int j, int ny,
+                                          bool fy, uint32_t e, const LevelSlots& s, const float (&val)[V]) {
+  const int mx = image_mask(i, nx, fx), my = image_mask(j, ny, fy);
+#pragma unroll 1
+  for (int a = 0; a < 3; ++a) {
+    if (!((mx >> a) & 1)) continue;
+    const int X = i + 3 + (a == 1 ? nx : (a == 2 ? -nx : 0));
+#pragma unroll 1
+    for (int b = 0; b < 3; ++b) {
+      if (!((my >> b) & 1)) continue;
+      const int Y = j + 3 + (b == 1 ? ny : (b == 2 ? -ny : 0));
+      const uint32_t o = (uint32_t)(X * sx + Y * sy) + e;
+      st_levels<V>(f, o, s, val);
+      if (ONW)
+        st_ghosts_w<V>(f, o, s, val);
+      else
+        st_ghosts<V>(f, o, s, val);
+    }
+  }
+}
+
+// MZ: the column spans several waves (nz > 64 V), whose edge lanes load their outer z
+// neighbours.
+template <int V, bool MZ>
+__global__ void __launch_bounds__(256) k_acoustic(Dims d, const float* __restrict__ rc, const float* __restrict__ pi0c,
+                                                  const float* __restrict__ u, const float* __restrict__ v,
+                                                  const float* __restrict__ w, const float* __restrict__ p,
+                                                  const float* __restrict__ ps, const float* __restrict__ ru,
+                                                  const float* __restrict__ rv, const float* __restrict__ rw,
+                                                  const float* __restrict__ tr, float* __restrict__ uo,
+                                                  float* __restrict__ vo, float* __restrict__ wo,
+                                                  float* __restrict__ po, float dts, int ax) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x;
+  const TileId tb = xcd_tile();
+  const int j = __builtin_amdgcn_readfirstlane(tb.x * (int)blockDim.y + (int)threadIdx.y);
+  const int nx = d.nx, ny = d.ny, nz = d.nz;
+  if (j >= ny) return;
+  const int x0 = tb.y * ax, x1 = min(x0 + ax, nx);
+  const int kl = (tb.z * 64 + lane) * V;         // the lane's first level
+  const int kc = min(kl, nz - 1);                // idle lanes repeat the last level
+  LevelSlots ls;
+  ls.n = min(max(nz - kl, 0), V);
+  ls.first = kl == 0;
+  ls.last = ls.n > 0 && kl + ls.n == nz;
+  const uint32_t eK = (uint32_t)(kc + 1);        // padded level of the lane's first level
+  const uint32_t ek = (uint32_t)min(kc, nz - V); // its level in an unpadded row
+  const bool past = (V == 2) && kc == nz - 1;
+  // column constants: reciprocal density, density at the lower w level, pi0 and its lower gradient
+  const float h = (float)(-kCp * 0.5);
+  float rr[V], ir[V], r8[V], pic[V], dpi[V];
+#pragma unroll
+  for (int q = 0; q < V; ++q) {
+    const int K = min(kc + q + 1, nz + 1);
+    rr[q] = rc[K];
+    ir[q] = 1.0f / rr[q];
+    r8[q] = 0.5f * (rc[K - 1] + rr[q]);
+    pic[q] = pi0c[K];
+    dpi[q] = (pic[q] - pi0c[K - 1]) * d.idz;
+  }
+  float r8e = 0.f, dpie = 0.f;   // of the level above the lane's last
+  if (MZ) {
+    const int K = min(kc + V + 1, nz + 1);
+    r8e = 0.5f * (rc[K - 1] + rc[K]);
+    dpie = (pi0c[K] - pi0c[K - 1]) * d.idz;
+  }
+  const bool edge = MZ && (lane == 0 || lane == 63);
+  const uint32_t eE = (uint32_t)(lane == 0 ? kc : min(kc + V + 1, nz + 1));
+  const uint32_t eW = (uint32_t)min(kc + V, nz);
+
+  const int syc = nz + 2, syw = nz + 3;
+  const int sxc = (ny + 6) * syc, sxv = (ny + 7) * syc, sxw = (ny + 6) * syw;
+  const int sxiu = ny * nz, sxiv = (ny + 1) * nz, sxiw = ny * (nz + 1);
+  // lane offsets within an x-plane: oc the cell rows j-1, j, j+1 (oc[1], oc[2] also the v
+  // faces j, j+1 and oc[1] the u row), ow the w row, oi the unpadded row and og rw's
+  const uint32_t oc[3] = {(uint32_t)((j + 2) * syc) + eK, (uint32_t)((j + 3) * syc) + eK, (uint32_t)((j + 4) * syc) + eK};
+  const uint32_t ow = (uint32_t)((j + 3) * syw) + eK;
+  const uint32_t oi = (uint32_t)(j * nz) + ek, oin = oi + (uint32_t)nz;
+  const uint32_t og = (uint32_t)(j * (nz + 1) + kc);
+  // the planes of x (cells, v, w) and of x + 1 (cells and u), advanced with the march
+  const float *pX = p + (long)(x0 + 3) * sxc, *tX = tr + (long)(x0 + 3) * sxc, *sX = ps + (long)(x0 + 3) * sxc;
+  const float *uX = u + (long)(x0 + 3) * sxc, *guX = ru + (long)x0 * sxiu;
+  const float *vX = v + (long)(x0 + 3) * sxv, *gvX = rv + (long)x0 * sxiv;
+  const float *wX = w + (long)(x0 + 3) * sxw, *gwX = rw + (long)x0 * sxiw;
+  float *poX = po + (long)(x0 + 3) * sxc, *uoX = uo + (long)(x0 + 3) * sxc, *voX = vo + (long)(x0 + 3) * sxv,
+        *woX = wo + (long)(x0 + 3) * sxw;
+
+  float P0[3][V], T0[3][V], S0[3][V];   // plane x, rows j-1, j, j+1
+  float ul[V], dl[V];                   // new u at face x and u dpi*/dx there
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    ld_levels<V>(pX, oc[r], P0[r]);
+    ld_levels<V>(tX, oc[r], T0[r]);
+    ld_levels<V>(sX, oc[r], S0[r]);
+  }
+  {
+    float pm[V], tm[V], sm[V], u0[V], g0[V];
+    ld_levels<V>(pX - sxc, oc[1], pm);
+    ld_levels<V>(tX - sxc, oc[1], tm);
+    ld_levels<V>(sX - sxc, oc[1], sm);
+    ld_levels<V>(uX, oc[1], u0);
+    ld_levels_in<V>(guX, oi, past, g0);
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      ul[q] = fmaf(fmaf(h * (T0[1][q] + tm[q]), (P0[1][q] - pm[q]) * d.idx, g0[q]), dts, u0[q]);
+      dl[q] = ul[q] * ((S0[1][q] - sm[q]) * d.idx);
+    }
+  }
+#pragma unroll 1
+  for (int x = x0; x < x1; ++x) {
+    float P1[3][V], T1[3][V], S1[3][V], uf[V], gu[V];
+    float vf[2][V], gv[2][V], wf[V], gw[V];
+    float pe, te, se, we, ge;
+    ld_levels<V>(vX, oc[1], vf[0]);
+    ld_levels<V>(vX, oc[2], vf[1]);
+    ld_levels_in<V>(gvX, oi, past, gv[0]);
+    ld_levels_in<V>(gvX, oin, past, gv[1]);
+    ld_levels<V>(wX, ow, wf);
+    ld_levels<V>(gwX, og, gw);
+    if (edge) {
+      pe = ld32(pX, oc[1] - eK + eE);
+      te = ld32(tX, oc[1] - eK + eE);
+      se = ld32(sX, oc[1] - eK + eE);
+      we = ld32(wX, ow - eK + eW + 1u);
+      ge = ld32(gwX, og - (uint32_t)kc + eW);
+    }
+    pX += sxc;
+    tX += sxc;
+    sX += sxc;
+    uX += sxc;
+    guX += sxiu;
+    vX += sxv;
+    gvX += sxiv;
+    wX += sxw;
+    gwX += sxiw;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      ld_levels<V>(pX, oc[r], P1[r]);
+      ld_levels<V>(tX, oc[r], T1[r]);
+      ld_levels<V>(sX, oc[r], S1[r]);
+    }
+    ld_levels<V>(uX, oc[1], uf);
+    ld_levels_in<V>(guX, oi, past, gu);
+    // y faces j, j+1
+    float vn[2][V], dv[2][V];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        vn[r][q] = fmaf(fmaf(h * (T0[r + 1][q] + T0[r][q]), (P0[r + 1][q] - P0[r][q]) * d.idy, gv[r][q]), dts, vf[r][q]);
+        dv[r][q] = vn[r][q] * ((S0[r + 1][q] - S0[r][q]) * d.idy);
+      }
+    const float(&pc)[V] = P0[1];
+    const float(&tc)[V] = T0[1];
+    const float(&sc)[V] = S0[1];
+    // lower z faces: new w, and its pi* term (half, then times the density)
+    float wn[V], a0[V], b0[V];
+    float pb = lane_below(pc[V - 1]), tb_ = lane_below(tc[V - 1]), sb = lane_below(sc[V - 1]);
+    if (MZ && lane == 0) {
+      pb = pe;
+      tb_ = te;
+      sb = se;
+    }
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      const float pl = q ? pc[0] : pb, tl = q ? tc[0] : tb_, sl = q ? sc[0] : sb;
+      const float pz = h * (tc[q] + tl) * ((pc[q] - pl) * d.idz);
+      const float wv = fmaf(pz + gw[q], dts, wf[q]);
+      const float dz = fmaf(sc[q] - sl, d.idz, dpi[q]);
+      const bool floor_ = q == 0 && kl == 0;
+      wn[q] = floor_ ? 0.0f : wv;
+      a0[q] = 0.5f * (floor_ ? 0.0f : wv * dz);
+      b0[q] = a0[q] * r8[q];
+    }
+    float wt = lane_above(wn[0]), bt = lane_above(b0[0]);
+    if (MZ && lane == 63) {
+      const float pz = h * (te + tc[V - 1]) * ((pe - pc[V - 1]) * d.idz);
+      wt = fmaf(pz + ge, dts, we);
+      bt = (0.5f * (wt * fmaf(se - sc[V - 1], d.idz, dpie))) * r8e;
+    }
+    float un[V], pn[V], us[V];
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      const bool lid = kl + q >= nz - 1;
+      const float w1 = lid ? 0.0f : (q < V - 1 ? wn[V - 1] : wt);
+      const float b1 = lid ? 0.0f : (q < V - 1 ? b0[V - 1] : bt);
+      un[q] = fmaf(fmaf(h * (T1[1][q] + tc[q]), (P1[1][q] - pc[q]) * d.idx, gu[q]), dts, uf[q]);
+      const float du = un[q] * ((S1[1][q] - sc[q]) * d.idx);
+      const float div = fmaf(w1 - wn[q], d.idz, fmaf(vn[1][q] - vn[0][q], d.idy, (un[q] - ul[q]) * d.idx));
+      const float z = quotient(fmaf(a0[q], r8[q], b1), rr[q], ir[q]);
+      const float advp = -(fmaf(0.5f, du + dl[q], 0.5f * (dv[1][q] + dv[0][q])) + z);
+      const float dpdt = fmaf((float)(-kRd / kCv), (pic[q] + sc[q]) * div, advp);
+      pn[q] = fmaf(1.1f * dpdt, dts, pc[q]);
+      us[q] = ul[q];
+      ul[q] = un[q];
+      dl[q] = du;
+    }
+    if (x >= 4 && x < nx - 3 && j >= 4 && j < ny - 3) {   // no periodic images
+      st_levels<V>(poX, oc[1], ls, pn);
+      st_levels<V>(uoX, oc[1], ls, us);
+      st_levels<V>(voX, oc[1], ls, vn[0]);
+      st_levels<V>(woX, ow, ls, wn);
+      if (ls.first || ls.last) {
+        st_ghosts<V>(poX, oc[1], ls, pn);
+        st_ghosts<V>(uoX, oc[1], ls, us);
+        st_ghosts<V>(voX, oc[1], ls, vn[0]);
+        st_ghosts_w<V>(woX, ow, ls, wn);
+      }
+    } else {
+      st_images<V, false>(po, sxc, syc, x, nx, false, j, ny, false, eK, ls, pn);
+      st_images<V, false>(uo, sxc, syc, x, nx, true, j, ny, false, eK, ls, us);
+      if (x == nx - 1) st_images<V, false>(uo, sxc, syc, nx, nx, true, j, ny, false, eK, ls, un);
+      st_images<V, false>(vo, sxv, syc, x, nx, false, j, ny, true, eK, ls, vn[0]);
+      if (j == ny - 1) st_images<V, false>(vo, sxv, syc, x, nx, false, ny, ny, true, eK, ls, vn[1]);
+      st_images<V, true>(wo, sxw, syw, x, nx, false, j, ny, false, eK, ls, wn);
+    }
+    poX += sxc;
+    uoX += sxc;
+    voX += sxv;
+    woX += sxw;
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        P0[r][q] = P1[r][q];
+        T0[r][q] = T1[r][q];
+        S0[r][q] = S1[r][q];
+      }
+  }
+}
+
+struct AcousticArgs {
+  const float *rc, *pi0, *u, *v, *w, *p, *ps, *ru, *rv, *rw, *tr;
+  float *uo, *vo, *wo, *po;
+  float dts;
+};
+
+template <int V>
+inline void launch_acoustic_v(const Dims& d, const AcousticArgs& a, hipStream_t st) {
+  const int chunks = (d.nz + 64 * V - 1) / (64 * V);
+  // Cells per wave along x: the prologue of a longer march is shared, as long as the launch
+  // keeps some 16 waves on every SIMD.  us per substep at ax = 1, 2, 4, 6: 96x96x48 11.2,
+  // 12.6, 16.2, 19.5; 128x128x64 15.6, 16.8, 19.4, 19.9; 181x147x70 38.0, 32.6, 31.6, 33.7;
+  // 192x160x96 43.6, 38.8, 40.9, 39.8; 240x240x120 111, 99, 97, 97; 256x256x128 129, 115, 113, 110.
+  const long waves = (long)d.nx * d.ny * chunks;
+  const int ax = (int)std::min(4L, std::max(1L, (waves + 8192) / 16384));
+  const dim3 g((d.ny + 3) / 4, (d.nx + ax - 1) / ax, chunks), b(64, 4, 1);
+  if (chunks == 1)
+    LEX_LAUNCH(KID_ACOUSTIC, (k_acoustic<V, false>), g, b, 0, st, d, a.rc, a.pi0, a.u, a.v, a.w, a.p, a.ps, a.ru, a.rv,
+               a.rw, a.tr, a.uo, a.vo, a.wo, a.po, a.dts, ax);
+  else
+    LEX_LAUNCH(KID_ACOUSTIC, (k_acoustic<V, true>), g, b, 0, st, d, a.rc, a.pi0, a.u, a.v, a.w, a.p, a.ps, a.ru, a.rv,
+               a.rw, a.tr, a.uo, a.vo, a.wo, a.po, a.dts, ax);
+}
+
+// One substep.  Two levels per lane where a column has more than one wave of them; us with
+// one and with two: 96x96x48 11.2 and 17.9, 128x128x64 15.6 and 26.6 (half the lanes idle);
+// 181x147x70 33.1 and 31.6, 240x240x120 120 and 97, 256x256x128 139 and 110.  The
+// cell-per-thread form took 13.9, 17.9, 35.8, 113 and 131; a copy of the thirteen fields of
+// 240x240x120 at 5 TB/s takes 72.
+inline void launch_acoustic(const Dims& d, const AcousticArgs& a, hipStream_t st) {
+  if (d.nz > 64)
+    launch_acoustic_v<2>(d, a, st);
+  else
+    launch_acoustic_v<1>(d, a, st);
+}
+
+}  // namespace lex

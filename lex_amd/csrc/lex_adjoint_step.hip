@@ -211,8 +211,8 @@ void rk3_forward_tape(const Dims& d, const O& o, const B& b, float* const* X0, c
       } else {
         acou_ptrs(ws + ac_off(L, s, t + 1), RL, out);
       }
-      hipLaunchKernelGGL(k_acoustic, cx.G(d.nz, d.ny, d.nx), cx.bk, 0, st, d, rc, b.pi0, in[0], in[1], in[2], in[3],
-                         src[4], ru, rv, rw, tr, out[0], out[1], out[2], out[3], dts);
+      launch_acoustic(d, AcousticArgs{rc, b.pi0, in[0], in[1], in[2], in[3], src[4], ru, rv, rw, tr, out[0], out[1],
+                                      out[2], out[3], dts}, st);
       for (int c = 0; c < 4; ++c) in[c] = out[c];
     }
     if (!fused) {

@@ -397,8 +397,7 @@ int lex_acoustic_substep(const lex_grid_t* g, const float* r, const float* pi0, 
   REQ(uo); REQ(vo); REQ(wo); REQ(po);
   if (uo == u || vo == v || wo == w || po == p) return fail(-1, "lex_acoustic_substep: outputs must not alias inputs%s");
   Dims d = mkdims(g);
-  hipLaunchKernelGGL(k_acoustic, grd(d.nz, d.ny, d.nx), blk(), 0, S(stream), d, r, pi0, u, v, w, p, ps, ru, rv, rw, tr,
-                     uo, vo, wo, po, dts);
+  launch_acoustic(d, AcousticArgs{r, pi0, u, v, w, p, ps, ru, rv, rw, tr, uo, vo, wo, po, dts}, S(stream));
   return check_launch("lex_acoustic_substep");
 }
 

@@ -495,6 +495,14 @@ __global__ void k_set_w_bc(Dims d, float* __restrict__ w) {
 // (u0/u1 lower/upper x face, ...), the rhs on those faces, the 7-point stencils of pi',
 // theta_rho and pi*, and the rho0 / pi0 column values at levels K-1, K, K+1.
 // ----------------------------------------------------------------------------------
+// x / r from the correctly rounded reciprocal ir of r: the product and one residual
+// correction, which is the correctly rounded quotient where nothing under- or overflows
+// (three operations instead of the ten of an IEEE division; r is a density).
+__device__ __forceinline__ float quotient(float x, float r, float ir) {
+  const float q = x * ir;
+  return fmaf(fmaf(-q, r, x), ir, q);
+}
+
 struct AcousticOut {
   float un0, un1, vn0, vn1, wn0, wn1, pn;
 };
@@ -550,54 +558,6 @@ __device__ __forceinline__ AcousticOut acoustic_cell(
 }
 
 // ----------------------------------------------------------------------------------
-// S1: one forward-backward acoustic substep (one_step_integration.py:528-553).
-// Reads u,v,w,pi' of the current substep, writes the next (halos filled, w BC set).
-// ----------------------------------------------------------------------------------
-__global__ void k_acoustic(Dims d, const float* __restrict__ rc, const float* __restrict__ pi0c,
-                           const float* __restrict__ u, const float* __restrict__ v, const float* __restrict__ w,
-                           const float* __restrict__ p, const float* __restrict__ ps, const float* __restrict__ ru,
-                           const float* __restrict__ rv, const float* __restrict__ rw, const float* __restrict__ tr,
-                           float* __restrict__ uo, float* __restrict__ vo, float* __restrict__ wo,
-                           float* __restrict__ po, float dts) {
-  const TileId tb = xcd_tile();
-  int k = tb.x * blockDim.x + threadIdx.x;
-  int j = tb.y * blockDim.y + threadIdx.y;
-  int i = tb.z;
-  if (k >= d.nz || j >= d.ny) return;
-  int I = i + 3, J = j + 3, K = k + 1;
-  const long c = ic(d, I, J, K);
-  const long sx = d.sxc(), sy = d.syc();
-  // Every operand is loaded unconditionally (all indices are inside the padded arrays,
-  // the w levels K and K+1 exist for K in 1..nz) so the loads issue back to back; the
-  // surface and lid cases are selected afterwards.
-  const float rcm = rc[K - 1], rcc = rc[K], rcp = rc[K + 1];
-  const float pim = pi0c[K - 1], pic = pi0c[K], pip = pi0c[K + 1];
-  const long cu = iu(d, I, J, K), cv = iv(d, I, J, K), cw = iw(d, I, J, K);
-  const long ou = ((long)i * d.ny + j) * d.nz + k, ov = ((long)i * (d.ny + 1) + j) * d.nz + k;
-  const long ow = ((long)i * d.ny + j) * (d.nz + 1) + k;
-  const float u0 = u[cu], u1 = u[cu + d.sxu()], v0 = v[cv], v1 = v[cv + d.syc()], w0 = w[cw], w1 = w[cw + 1];
-  const float ru0 = ru[ou], ru1 = ru[ou + (long)d.ny * d.nz], rv0 = rv[ov], rv1 = rv[ov + d.nz];
-  const float rw0 = rw[ow], rw1 = rw[ow + 1];
-  const float pc = p[c], pxm = p[c - sx], pxp = p[c + sx], pym = p[c - sy], pyp = p[c + sy], pzm = p[c - 1],
-              pzp = p[c + 1];
-  const float tc = tr[c], txm = tr[c - sx], txp = tr[c + sx], tym = tr[c - sy], typ = tr[c + sy],
-              tzm = tr[c - 1], tzp = tr[c + 1];
-  const float sc = ps[c], sxm = ps[c - sx], sxp = ps[c + sx], sym = ps[c - sy], syp = ps[c + sy],
-              szm = ps[c - 1], szp = ps[c + 1];
-  const AcousticOut o = acoustic_cell(d, k, u0, u1, v0, v1, w0, w1, ru0, ru1, rv0, rv1, rw0, rw1, pc, pxm, pxp, pym,
-                                      pyp, pzm, pzp, tc, txm, txp, tym, typ, tzm, tzp, sc, sxm, sxp, sym, syp, szm, szp,
-                                      rcm, rcc, rcp, pim, pic, pip, dts);
-  const float pn = o.pn, un0 = o.un0, un1 = o.un1, vn0 = o.vn0, vn1 = o.vn1, wn0 = o.wn0, wn1 = o.wn1;
-  store_c_fast(d, po, i, j, k, pn);
-  store_u_fast(d, uo, i, j, k, un0);
-  if (i == d.nx - 1) store_u(d, uo, d.nx, j, k, un1);
-  store_v_fast(d, vo, i, j, k, vn0);
-  if (j == d.ny - 1) store_v(d, vo, i, d.ny, k, vn1);
-  store_w_fast(d, wo, i, j, k, wn0);
-  if (k == d.nz - 1) store_w(d, wo, i, j, d.nz, wn1);
-}
-
-// ----------------------------------------------------------------------------------
 // k_acoustic2: two consecutive S1 substeps in one launch (the same arithmetic as two
 // k_acoustic launches, acoustic_cell for each).  A workgroup owns whole z-columns of a
 // strip of R-2 rows in y and marches `ax` cells along x.  Each thread takes one
@@ -619,6 +579,14 @@ inline int acoustic2_rows(const Dims& d) {
   return r > kA2Rows ? kA2Rows : r;
 }
 inline bool acoustic2_ok(const Dims& d) { return acoustic2_rows(d) >= 4; }
+// Whether two substeps are faster in one launch than in two: only where the thirteen fields
+// of a substep do not fit the 256 MB last-level cache with room to spare, so that the second
+// substep's operands would come from HBM again.  Pair against two substeps, us: 96x96x48 29
+// and 22, 128x128x64 38 and 31, 181x147x70 84 and 63, 192x160x96 96 and 78, 240x240x120 191
+// and 193, 256x256x128 193 and 225.
+inline bool acoustic2_pays(const Dims& d) {
+  return acoustic2_ok(d) && (long)d.nx * d.ny * d.nz >= 6500000L;
+}
 inline size_t acoustic2_lds(const Dims& d) {
   return (size_t)3 * acoustic2_rows(d) * (acoustic2_lanes(d) + 2) * sizeof(float);
 }

@@ -9,6 +9,7 @@
 #include "lex_common.hpp"
 #include "lex_prof.hpp"
 #include "lex_fused.hip"
+#include "lex_acoustic_rows.hip"
 #include "lex_acoustic_vi.hip"
 #include "lex_surface.hip"
 
@@ -484,7 +485,7 @@ int rk3_step(const Dims& d, const O& o, const B& b, float* const* state, char* w
     }
     float* in[4] = {X0[1], X0[2], X0[3], X0[4]};
     // the fused path advances two substeps per launch while two remain
-    const bool pairs = (o.solver != 3) && (o.impl == 0) && acoustic2_ok(d);
+    const bool pairs = (o.solver != 3) && (o.impl == 0) && acoustic2_pays(d);
     for (int t = 0; t < nsub;) {
       const int tn = t + ((pairs && t + 1 < nsub) ? 2 : 1);
       float* out[4];
@@ -509,8 +510,8 @@ int rk3_step(const Dims& d, const O& o, const B& b, float* const* state, char* w
                    acoustic2_lds(d), st, d, rc, b.pi0, in[0], in[1], in[2], in[3], src[4], ru, rv, rw, tr, out[0],
                    out[1], out[2], out[3], dts, acoustic2_ax(d));
       } else {
-        LEX_LAUNCH(KID_ACOUSTIC, k_acoustic, G(d.nz, d.ny, d.nx), bk, 0, st, d, rc, b.pi0, in[0], in[1], in[2], in[3],
-                   src[4], ru, rv, rw, tr, out[0], out[1], out[2], out[3], dts);
+        launch_acoustic(d, AcousticArgs{rc, b.pi0, in[0], in[1], in[2], in[3], src[4], ru, rv, rw, tr, out[0], out[1],
+                                        out[2], out[3], dts}, st);
       }
       if (alias) {
         const size_t ns[4] = {L.nu, L.nv, L.nw, L.nc};

@@ -35,3 +35,36 @@ def test_stage_tiles_equal_per_operator_kernels(shape, passive):
         assert np.isfinite(b).all()
         ulp = float(np.spacing(np.float32(np.abs(b).max())))
         assert np.max(np.abs(a - b)) <= 64 * ulp, (q, np.max(np.abs(a - b)) / ulp)
+
+
+# one and two levels per lane, columns of one wave and of several with one level left over,
+# even and odd nz, marches of one and of several cells
+@pytest.mark.parametrize("shape", [(8, 9, 24), (17, 9, 64), (9, 7, 65), (33, 18, 128), (6, 6, 129), (20, 21, 200),
+                                   (161, 120, 73)], ids=str)
+def test_acoustic_substep_against_oracle(shape):
+    """One substep against the FP64 oracle, the input's ghosts not periodic images (an initial
+    state's need not be); error within 8x the FP32 oracle's own, as for the other operators."""
+    import torch
+    from lex_amd import _lib
+    from oracle import lex_oracle as o
+    from tests._helpers import check_fp32
+    nx, ny, nz = shape
+    gr, phys, base = random_state(nx, ny, nz, seed=5, vel=2.0)
+    rng = np.random.default_rng(7)
+    th, u, v, w, p = phys[:5]
+    p = np.asarray(p + rng.normal(0, 1e-5, p.shape), np.float32)
+    ps = np.asarray(p + rng.normal(0, 1e-6, p.shape), np.float32)
+    u, v, w, th = (np.asarray(a, np.float32) for a in (u, v, w, th))
+    ru, rv, rw = (np.asarray(rng.normal(0, 1e-2, s), np.float32)
+                  for s in ((nx + 1, ny, nz), (nx, ny + 1, nz), (nx, ny, nz + 1)))
+    rho, pi0 = (np.asarray(base[q], np.float32) for q in (1, 3))
+    ref = []
+    for dt in (np.float64, np.float32):
+        f = lambda a: np.asarray(a, dt)  # noqa: E731
+        ref.append(o.sound_rk_step(f(u), f(v), f(w), f(pi0), f(p), f(ps), f(ru), f(rv), f(rw), f(th), f(rho), 1, 0.1, gr))
+    ins = [to_dev(a) for a in (rho[3, 3], pi0[3, 3], u, v, w, p, ps, ru, rv, rw, th)]
+    out = [torch.full_like(t, float("nan")) for t in ins[2:6]]
+    g = _lib.grid(nx, ny, nz, gr.dx, gr.dy, gr.dz)
+    _lib.call("lex_acoustic_substep", g, *[_lib.ptr(t) for t in ins], 0.1, *[_lib.ptr(t) for t in out], _lib.stream())
+    for name, got, r64, r32 in zip("u v w p".split(), out, *ref):
+        check_fp32(from_dev(got), r64, r32, name)
