@@ -116,6 +116,9 @@ struct BicgState {
   int k_final;   // exit code (iterations, or -10 / -11 on breakdown)
   int maxiter;
   int pad;
+  // what block 0 of one kernel hands to the next, so that each sum is reduced once: K1
+  // writes atol2 (iteration 0) and rho_new, K2 alpha
+  double atol2, rho_new, alpha;
 };
 static_assert(sizeof(BicgState) <= 256, "BiCGSTAB loop state fits its 256-byte slot");
 
@@ -127,20 +130,15 @@ constexpr int kBicgCellsPerThread = 2;   // grid size (1-16 measured within 15 %
 constexpr int kBicgSlots = 1 + 4 + 1 + 3;
 constexpr size_t kBicgPartialBytes = (size_t)kBicgSlots * kBicgBlocks * sizeof(double);
 struct BicgPartials {
-  double* bb;      // [nb]
-  double* rr[2];   // [2][nb] by parity: r.r, then rhat.r
-  double* rq;      // [nb]
-  double* ts;      // [3][nb]: t.s, t.t, s.s
+  double* base;
+  // Addresses by arithmetic: an array of pointers indexed at run time would go through LDS,
+  // and the kernel would read its dispatch packet from host memory for the workgroup size
+  // (10 us of each launch's 20).
+  __host__ __device__ double* bb() const { return base; }                                    // [nb]
+  __host__ __device__ double* rr(int par) const { return base + (1 + 2 * par) * kBicgBlocks; }  // [2][nb]: r.r, rhat.r
+  __host__ __device__ double* rq() const { return base + 5 * kBicgBlocks; }                  // [nb]
+  __host__ __device__ double* ts() const { return base + 6 * kBicgBlocks; }                  // [3][nb]: t.s, t.t, s.s
 };
-__host__ __device__ inline BicgPartials bicg_partials(double* base) {
-  BicgPartials P;
-  P.bb = base;
-  P.rr[0] = base + kBicgBlocks;
-  P.rr[1] = base + 3 * kBicgBlocks;
-  P.rq = base + 5 * kBicgBlocks;
-  P.ts = base + 6 * kBicgBlocks;
-  return P;
-}
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -162,30 +160,51 @@ __device__ __forceinline__ void block_sum_all(const double (&v)[NV], double (&ou
 #pragma unroll
   for (int q = 0; q < NV; ++q) {
     double t = 0.0;
+#pragma unroll
     for (int w = 0; w < kBicgThreads / 64; ++w) t += sh[q][w];
     out[q] = t;
   }
-  __syncthreads();
 }
 
-// Sum of NV partial arrays (stride kBicgBlocks, nb entries each) in a fixed order,
-// returned to every thread of the block.
+// This thread's share of NV partial arrays (nb entries each, strided over the block), in a
+// fixed order.  Every entry of every array is requested before the first is needed, so the
+// prologue of a kernel waits once for what other XCDs wrote, not once per array.
 template <int NV>
-__device__ __forceinline__ void sum_partials(const double* __restrict__ P, int nb, double (&tot)[NV]) {
-  double v[NV];
+struct PartialShare {
+  static constexpr int kEach = kBicgBlocks / kBicgThreads;
+  double v[NV][kEach];
+  __device__ __forceinline__ void request(const double* const (&P)[NV], int nb) {
 #pragma unroll
-  for (int q = 0; q < NV; ++q) {
-    double s = 0.0;
-    for (int b = threadIdx.x; b < nb; b += kBicgThreads) s += P[q * kBicgBlocks + b];
-    v[q] = s;
+    for (int e = 0; e < kEach; ++e) {
+      const int b = threadIdx.x + e * kBicgThreads;
+      const uint32_t c = (uint32_t)min(b, nb - 1);   // loads without a branch per thread
+#pragma unroll
+      for (int q = 0; q < NV; ++q) {
+        v[q][e] = 0.0;
+        if (e * kBicgThreads < nb) {
+          const double x = P[q][c];
+          v[q][e] = b < nb ? x : 0.0;
+        }
+      }
+    }
   }
-  block_sum_all<NV>(v, tot);
-}
+  __device__ __forceinline__ void sum(double (&tot)[NV]) const {
+    double s[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      s[q] = 0.0;
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) s[q] += v[q][e];
+    }
+    block_sum_all<NV>(s, tot);
+  }
+};
 
 // Write this block's sums of NV per-thread values to P[q * kBicgBlocks + blockIdx.x].
 template <int NV>
 __device__ __forceinline__ void put_partials(const double (&acc)[NV], double* __restrict__ P) {
   double tot[NV];
+  __syncthreads();   // the prologue's sums have been read
   block_sum_all<NV>(acc, tot);
   if (threadIdx.x == 0) {
 #pragma unroll
@@ -193,53 +212,51 @@ __device__ __forceinline__ void put_partials(const double (&acc)[NV], double* __
   }
 }
 
-// Interior cell (i, j, k) of the unpadded linear index t (x slowest, z fastest).
-__device__ __forceinline__ void cell_of(const Dims& d, long t, int& i, int& j, int& k) {
-  const long jt = t / d.nz;
-  k = (int)(t - jt * d.nz);
-  i = (int)(jt / d.ny);
-  j = (int)(jt - (long)i * d.ny);
-}
-
-// laplace_of_pressure (pressure_equations.py:8-48) at (i, j, k) of a vector given by
-// F(offset) on the unpadded (nx, ny, nz) layout: periodic in x and y, z clamped to the
-// end levels; arithmetic in the order of matvec_point.
-template <class F>
-__device__ __forceinline__ float matvec_at(const Dims& d, const float* __restrict__ rtt, int i, int j, int k, long t,
-                                           const F& X, float& xc) {
-  const long syz = (long)d.ny * d.nz;
-  const long oxm = (i == 0) ? t + (long)(d.nx - 1) * syz : t - syz;
-  const long oxp = (i == d.nx - 1) ? t - (long)(d.nx - 1) * syz : t + syz;
-  const long oym = (j == 0) ? t + (long)(d.ny - 1) * d.nz : t - d.nz;
-  const long oyp = (j == d.ny - 1) ? t - (long)(d.ny - 1) * d.nz : t + d.nz;
-  const long ozm = (k == 0) ? t : t - 1;
-  const long ozp = (k == d.nz - 1) ? t : t + 1;
-  const long cc = ic(d, i + 3, j + 3, k + 1);
-  const long sx = d.sxc(), sy = d.syc();
-  xc = X(t);
-  float px0 = 0.5f * (rtt[cc] + rtt[cc - sx]) * ((xc - X(oxm)) * d.idx);
-  float px1 = 0.5f * (rtt[cc + sx] + rtt[cc]) * ((X(oxp) - xc) * d.idx);
-  float py0 = 0.5f * (rtt[cc] + rtt[cc - sy]) * ((xc - X(oym)) * d.idy);
-  float py1 = 0.5f * (rtt[cc + sy] + rtt[cc]) * ((X(oyp) - xc) * d.idy);
-  float pz0 = (k == 0) ? rtt[cc - 1] : 0.5f * (rtt[cc] + rtt[cc - 1]) * ((xc - X(ozm)) * d.idz);
-  float pz1 = (k == d.nz - 1) ? rtt[cc + 1] : 0.5f * (rtt[cc + 1] + rtt[cc]) * ((X(ozp) - xc) * d.idz);
-  return (float)kCp * ((px1 - px0) * d.idx + (py1 - py0) * d.idy + (pz1 - pz0) * d.idz);
-}
-
-// Scalars every kernel of iteration `it` derives from the partials: |r|^2 and rhat.r
-// of the iteration's starting residual, and atol^2.
-struct BicgTop {
-  double rr, rho_new, atol2;
+// The pressure operator's stencil at the unpadded linear index t (x slowest, z fastest): the
+// offsets of the seven points in an unpadded vector (periodic in x and y, z clamped to the
+// end levels) and the cell's offset in the padded rtt.
+struct Stencil {
+  uint32_t c, xm, xp, ym, yp, zm, zp, rc;
+  bool first, last;   // lowest / highest level
 };
-__device__ __forceinline__ BicgTop bicg_top(const BicgPartials& P, int nb, int it, double tol, double atol) {
-  double a[2], bb[1];
-  sum_partials<2>(P.rr[(it + 1) & 1], nb, a);
-  sum_partials<1>(P.bb, nb, bb);
-  BicgTop t;
-  t.rr = a[0];
-  t.rho_new = a[1];
-  t.atol2 = fmax(tol * tol * bb[0], atol * atol);
-  return t;
+__device__ __forceinline__ Stencil stencil_at(const Dims& d, uint32_t t) {
+  const uint32_t nz = d.nz, ny = d.ny, nx = d.nx;
+  const uint32_t jt = t / nz, k = t - jt * nz, i = jt / ny, j = jt - i * ny, syz = ny * nz;
+  Stencil s;
+  s.c = t;
+  s.xm = (i == 0) ? t + (nx - 1) * syz : t - syz;
+  s.xp = (i == nx - 1) ? t - (nx - 1) * syz : t + syz;
+  s.ym = (j == 0) ? t + (ny - 1) * nz : t - nz;
+  s.yp = (j == ny - 1) ? t - (ny - 1) * nz : t + nz;
+  s.first = k == 0;
+  s.last = k == nz - 1;
+  s.zm = s.first ? t : t - 1;
+  s.zp = s.last ? t : t + 1;
+  s.rc = ((i + 3) * (ny + 6) + j + 3) * (nz + 2) + k + 1;
+  return s;
+}
+// A value per stencil point.
+struct Seven {
+  float c, xm, xp, ym, yp, zm, zp;
+};
+__device__ __forceinline__ Seven load7(const float* __restrict__ a, const Stencil& s) {
+  return Seven{ld32(a, s.c), ld32(a, s.xm), ld32(a, s.xp), ld32(a, s.ym), ld32(a, s.yp), ld32(a, s.zm), ld32(a, s.zp)};
+}
+__device__ __forceinline__ Seven load_rtt(const Dims& d, const float* __restrict__ rtt, const Stencil& s) {
+  const uint32_t sy = d.nz + 2, sx = (d.ny + 6) * sy;
+  return Seven{ld32(rtt, s.rc), ld32(rtt, s.rc - sx), ld32(rtt, s.rc + sx), ld32(rtt, s.rc - sy), ld32(rtt, s.rc + sy),
+               ld32(rtt, s.rc - 1), ld32(rtt, s.rc + 1)};
+}
+// laplace_of_pressure (pressure_equations.py:8-48) from the stencil values of rtt and x;
+// arithmetic in the order of matvec_point.
+__device__ __forceinline__ float matvec7(const Dims& d, const Stencil& s, const Seven& r, const Seven& x) {
+  float px0 = 0.5f * (r.c + r.xm) * ((x.c - x.xm) * d.idx);
+  float px1 = 0.5f * (r.xp + r.c) * ((x.xp - x.c) * d.idx);
+  float py0 = 0.5f * (r.c + r.ym) * ((x.c - x.ym) * d.idy);
+  float py1 = 0.5f * (r.yp + r.c) * ((x.yp - x.c) * d.idy);
+  float pz0 = s.first ? r.zm : 0.5f * (r.c + r.zm) * ((x.c - x.zm) * d.idz);
+  float pz1 = s.last ? r.zp : 0.5f * (r.zp + r.c) * ((x.zp - x.c) * d.idz);
+  return (float)kCp * ((px1 - px0) * d.idx + (py1 - py0) * d.idy + (pz1 - pz0) * d.idz);
 }
 
 // clear the loop state (a kernel, not a memset, so the solve can be graph-captured)
@@ -262,26 +279,40 @@ __global__ void __launch_bounds__(kBicgThreads) k_bicg_init(Dims d, const float*
                                                            float* __restrict__ x, float* __restrict__ r,
                                                            float* __restrict__ rhat, float* __restrict__ p,
                                                            float* __restrict__ q, double* __restrict__ partials) {
-  const BicgPartials P = bicg_partials(partials);
-  const long n = (long)d.nx * d.ny * d.nz;
+  const BicgPartials P{partials};
+  const uint32_t n = (uint32_t)d.nx * d.ny * d.nz, stride = gridDim.x * blockDim.x;
   double acc[2] = {0.0, 0.0};
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-    int i, j, k;
-    cell_of(d, t, i, j, k);
-    float ri = b[t] - matvec_point(d, rtt, x0, i, j, k);
-    x[t] = x0[t];
+  for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += stride) {
+    const Stencil s = stencil_at(d, t);
+    const Seven xv = load7(x0, s);
+    const float bt = b[t];
+    const float ri = bt - matvec7(d, s, load_rtt(d, rtt, s), xv);
+    x[t] = xv.c;
     r[t] = ri;
     rhat[t] = ri;
     p[t] = ri;
     q[t] = ri;
-    acc[0] += (double)b[t] * b[t];
+    acc[0] += (double)bt * bt;
     acc[1] += (double)ri * ri;
   }
-  double bb[1] = {acc[0]};
-  double rr[2] = {acc[1], acc[1]};
-  put_partials<1>(bb, P.bb);
-  put_partials<2>(rr, P.rr[1]);
+  double v[3] = {acc[0], acc[1], acc[1]};
+  double tot[3];
+  block_sum_all<3>(v, tot);
+  if (threadIdx.x == 0) {
+    P.bb()[blockIdx.x] = tot[0];
+    P.rr(1)[blockIdx.x] = tot[1];
+    P.rr(1)[kBicgBlocks + blockIdx.x] = tot[2];
+  }
 }
+
+// What the three kernels of an iteration share.  They are latency-bound: the fields of the
+// sizes solved here stay in the caches and a kernel is one chain of launch, loads, block
+// reduction, arithmetic, block reduction.  So everything a thread reads - its first two
+// cells' operands, the partial sums, the loop state - is requested before the first wait,
+// and each sum is reduced by one kernel only.  64x64x40, us per launch of K1, K2, K3: 6.2, 5.2, 5.8
+// (20.3, 20.7, 20.6 with a wait per array and per cell, 64-bit indices and a pointer table
+// in LDS; an empty kernel of this grid takes 2.7).
+constexpr int kBicgAhead = 2;   // cells of a thread whose operands are requested up front
 
 // K1 of iteration it: the loop test; beta; p' = r + beta (p - omega q) (recomputed on
 // the stencil's points); q' = A(p'); partials rhat.q'
@@ -291,102 +322,187 @@ __global__ void __launch_bounds__(kBicgThreads) k_bicg_pq(Dims d, const float* _
                                                          float* __restrict__ pn, float* __restrict__ qn,
                                                          double* __restrict__ partials, BicgState* st, int it, int nb,
                                                          double tol, double atol) {
-  if (st->done) return;
-  const BicgPartials P = bicg_partials(partials);
-  const BicgTop top = bicg_top(P, nb, it, tol, atol);
+  const uint32_t n = (uint32_t)d.nx * d.ny * d.nz, stride = gridDim.x * blockDim.x;
+  const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x;
+  const BicgPartials P{partials};
+  const int done = st->done, maxiter = st->maxiter;
   const BicgScalars sc = st->s[it & 1];
-  if (!(top.rr > top.atol2 && sc.k < st->maxiter && sc.k >= 0)) {
+  const double* const rr = P.rr((it + 1) & 1);
+  const double atol2_prev = st->atol2;
+  PartialShare<2> sh;
+  PartialShare<1> shb;
+  sh.request({rr, rr + kBicgBlocks}, nb);
+  if (it == 0) shb.request({P.bb()}, nb);
+  Stencil s[kBicgAhead];
+  Seven rt[kBicgAhead], rv[kBicgAhead], pv[kBicgAhead], qv[kBicgAhead];
+  float rh[kBicgAhead];
+  auto fetch = [&](int e, uint32_t t) {
+    s[e] = stencil_at(d, t);
+    rt[e] = load_rtt(d, rtt, s[e]);
+    rv[e] = load7(r, s[e]);
+    pv[e] = load7(p, s[e]);
+    qv[e] = load7(q, s[e]);
+    rh[e] = ld32(rhat, t);
+  };
+#pragma unroll
+  for (int e = 0; e < kBicgAhead; ++e) fetch(e, min(t0 + e * stride, n - 1));
+  if (done) return;
+  double a[2];
+  sh.sum(a);
+  const double rho_new = a[1];
+  double atol2 = atol2_prev;
+  if (it == 0) {
+    double bb[1];
+    shb.sum(bb);
+    atol2 = fmax(tol * tol * bb[0], atol * atol);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (it == 0) st->atol2 = atol2;
+    st->rho_new = rho_new;
+  }
+  if (!(a[0] > atol2 && sc.k < maxiter && sc.k >= 0)) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       st->done = 1;
       st->k_final = sc.k;
     }
     return;
   }
-  const double beta_d = top.rho_new / sc.rho * sc.alpha / sc.omega;
+  const double beta_d = rho_new / sc.rho * sc.alpha / sc.omega;
   const float beta = (float)beta_d, om = (float)sc.omega;
-  const long n = (long)d.nx * d.ny * d.nz;
   double acc[1] = {0.0};
-  auto Pv = [&](long o) { return r[o] + beta * (p[o] - om * q[o]); };
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-    int i, j, k;
-    cell_of(d, t, i, j, k);
-    float xc;
-    const float qv = matvec_at(d, rtt, i, j, k, t, Pv, xc);
-    pn[t] = xc;
-    qn[t] = qv;
-    acc[0] += (double)rhat[t] * qv;
+  auto cell = [&](int e, uint32_t t) {
+    auto Pv = [&](float ro, float po, float qo) { return ro + beta * (po - om * qo); };
+    const Seven& R = rv[e];
+    const Seven& Q = pv[e];
+    const Seven& W = qv[e];
+    const Seven x{Pv(R.c, Q.c, W.c),    Pv(R.xm, Q.xm, W.xm), Pv(R.xp, Q.xp, W.xp), Pv(R.ym, Q.ym, W.ym),
+                  Pv(R.yp, Q.yp, W.yp), Pv(R.zm, Q.zm, W.zm), Pv(R.zp, Q.zp, W.zp)};
+    const float y = matvec7(d, s[e], rt[e], x);
+    pn[t] = x.c;
+    qn[t] = y;
+    acc[0] += (double)rh[e] * y;
+  };
+#pragma unroll
+  for (int e = 0; e < kBicgAhead; ++e)
+    if (t0 + e * stride < n) cell(e, t0 + e * stride);
+  for (uint32_t t = t0 + kBicgAhead * stride; t < n; t += stride) {
+    fetch(0, t);
+    cell(0, t);
   }
-  put_partials<1>(acc, P.rq);
+  put_partials<1>(acc, P.rq());
 }
 
 // K2: alpha = rho_new / rhat.q; s = r - alpha q (recomputed on the stencil), t = A(s);
 // partials t.s, t.t, s.s
 __global__ void __launch_bounds__(kBicgThreads) k_bicg_st(Dims d, const float* __restrict__ rtt,
                                                          const float* __restrict__ r, const float* __restrict__ q,
-                                                         float* __restrict__ s, float* __restrict__ tv,
-                                                         double* __restrict__ partials, BicgState* st, int it, int nb,
-                                                         double tol, double atol) {
-  if (st->done) return;
-  const BicgPartials P = bicg_partials(partials);
-  const BicgTop top = bicg_top(P, nb, it, tol, atol);
+                                                         float* __restrict__ sv, float* __restrict__ tv,
+                                                         double* __restrict__ partials, BicgState* st, int nb) {
+  const uint32_t n = (uint32_t)d.nx * d.ny * d.nz, stride = gridDim.x * blockDim.x;
+  const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x;
+  const BicgPartials P{partials};
+  const int done = st->done;
+  const double rho_new = st->rho_new;
+  PartialShare<1> sh;
+  sh.request({P.rq()}, nb);
+  Stencil s[kBicgAhead];
+  Seven rt[kBicgAhead], rv[kBicgAhead], qv[kBicgAhead];
+  auto fetch = [&](int e, uint32_t t) {
+    s[e] = stencil_at(d, t);
+    rt[e] = load_rtt(d, rtt, s[e]);
+    rv[e] = load7(r, s[e]);
+    qv[e] = load7(q, s[e]);
+  };
+#pragma unroll
+  for (int e = 0; e < kBicgAhead; ++e) fetch(e, min(t0 + e * stride, n - 1));
+  if (done) return;
   double rq[1];
-  sum_partials<1>(P.rq, nb, rq);
-  const float al = (float)(top.rho_new / rq[0]);
-  const long n = (long)d.nx * d.ny * d.nz;
+  sh.sum(rq);
+  const double alpha = rho_new / rq[0];
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->alpha = alpha;
+  const float al = (float)alpha;
   double acc[3] = {0.0, 0.0, 0.0};
-  auto Sv = [&](long o) { return r[o] - al * q[o]; };
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-    int i, j, k;
-    cell_of(d, t, i, j, k);
-    float xc;
-    const float tt = matvec_at(d, rtt, i, j, k, t, Sv, xc);
-    s[t] = xc;
-    tv[t] = tt;
-    acc[0] += (double)tt * xc;
-    acc[1] += (double)tt * tt;
-    acc[2] += (double)xc * xc;
+  auto cell = [&](int e, uint32_t t) {
+    auto Sv = [&](float ro, float qo) { return ro - al * qo; };
+    const Seven& R = rv[e];
+    const Seven& Q = qv[e];
+    const Seven x{Sv(R.c, Q.c),   Sv(R.xm, Q.xm), Sv(R.xp, Q.xp), Sv(R.ym, Q.ym),
+                  Sv(R.yp, Q.yp), Sv(R.zm, Q.zm), Sv(R.zp, Q.zp)};
+    const float y = matvec7(d, s[e], rt[e], x);
+    sv[t] = x.c;
+    tv[t] = y;
+    acc[0] += (double)y * x.c;
+    acc[1] += (double)y * y;
+    acc[2] += (double)x.c * x.c;
+  };
+#pragma unroll
+  for (int e = 0; e < kBicgAhead; ++e)
+    if (t0 + e * stride < n) cell(e, t0 + e * stride);
+  for (uint32_t t = t0 + kBicgAhead * stride; t < n; t += stride) {
+    fetch(0, t);
+    cell(0, t);
   }
-  put_partials<3>(acc, P.ts);
+  put_partials<3>(acc, P.ts());
 }
 
 // K3: omega = t.s / t.t; x, r updates (early exit when |s|^2 < atol^2); partials r.r,
 // rhat.r for the next iteration; block 0 advances the recurrence scalars
-__global__ void __launch_bounds__(kBicgThreads) k_bicg_xr(long n, const float* __restrict__ p,
-                                                         const float* __restrict__ s, const float* __restrict__ tv,
+__global__ void __launch_bounds__(kBicgThreads) k_bicg_xr(long nl, const float* __restrict__ p,
+                                                         const float* __restrict__ sv, const float* __restrict__ tv,
                                                          const float* __restrict__ rhat, float* __restrict__ x,
                                                          float* __restrict__ r, double* __restrict__ partials,
-                                                         BicgState* st, int it, int nb, double tol, double atol) {
-  if (st->done) return;
-  const BicgPartials P = bicg_partials(partials);
-  const BicgTop top = bicg_top(P, nb, it, tol, atol);
-  double rq[1], ts[3];
-  sum_partials<1>(P.rq, nb, rq);
-  sum_partials<3>(P.ts, nb, ts);
-  const double alpha_new = top.rho_new / rq[0];
-  const double omega_new = ts[0] / ts[1];
-  const bool early = ts[2] < top.atol2;
+                                                         BicgState* st, int it, int nb) {
+  const uint32_t n = (uint32_t)nl, stride = gridDim.x * blockDim.x;
+  const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x;
+  const BicgPartials P{partials};
+  const int done = st->done;
+  const int k0 = st->s[it & 1].k;
+  const double rho_new = st->rho_new, alpha_new = st->alpha, atol2 = st->atol2;
+  PartialShare<3> sh;
+  sh.request({P.ts(), P.ts() + kBicgBlocks, P.ts() + 2 * kBicgBlocks}, nb);
+  float xv[kBicgAhead], pv[kBicgAhead], ss[kBicgAhead], tt[kBicgAhead], rh[kBicgAhead];
+  auto fetch = [&](int e, uint32_t t) {
+    xv[e] = ld32(x, t);
+    pv[e] = ld32(p, t);
+    ss[e] = ld32(sv, t);
+    tt[e] = ld32(tv, t);
+    rh[e] = ld32(rhat, t);
+  };
+#pragma unroll
+  for (int e = 0; e < kBicgAhead; ++e) fetch(e, min(t0 + e * stride, n - 1));
+  if (done) return;
+  double a[3];   // t.s, t.t, s.s
+  sh.sum(a);
+  const double omega_new = a[0] / a[1];
+  const bool early = a[2] < atol2;
   const float al = (float)alpha_new, om = (float)omega_new;
   double acc[2] = {0.0, 0.0};
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
+  auto cell = [&](int e, uint32_t t) {
     float rn;
     if (early) {
-      x[t] = x[t] + al * p[t];
-      rn = s[t];
+      x[t] = xv[e] + al * pv[e];
+      rn = ss[e];
     } else {
-      x[t] = x[t] + (al * p[t] + om * s[t]);
-      rn = s[t] - om * tv[t];
+      x[t] = xv[e] + (al * pv[e] + om * ss[e]);
+      rn = ss[e] - om * tt[e];
     }
     r[t] = rn;
     acc[0] += (double)rn * rn;
-    acc[1] += (double)rhat[t] * rn;
+    acc[1] += (double)rh[e] * rn;
+  };
+#pragma unroll
+  for (int e = 0; e < kBicgAhead; ++e)
+    if (t0 + e * stride < n) cell(e, t0 + e * stride);
+  for (uint32_t t = t0 + kBicgAhead * stride; t < n; t += stride) {
+    fetch(0, t);
+    cell(0, t);
   }
-  put_partials<2>(acc, P.rr[it & 1]);
+  put_partials<2>(acc, P.rr(it & 1));
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    const BicgScalars sc = st->s[it & 1];
-    int kn = (omega_new == 0.0 || alpha_new == 0.0) ? -11 : sc.k + 1;
-    if (top.rho_new == 0.0) kn = -10;
+    int kn = (omega_new == 0.0 || alpha_new == 0.0) ? -11 : k0 + 1;
+    if (rho_new == 0.0) kn = -10;
     BicgScalars nx;
-    nx.rho = top.rho_new;
+    nx.rho = rho_new;
     nx.alpha = alpha_new;
     nx.omega = omega_new;
     nx.k = kn;

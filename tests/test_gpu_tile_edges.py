@@ -68,3 +68,35 @@ def test_acoustic_substep_against_oracle(shape):
     _lib.call("lex_acoustic_substep", g, *[_lib.ptr(t) for t in ins], 0.1, *[_lib.ptr(t) for t in out], _lib.stream())
     for name, got, r64, r32 in zip("u v w p".split(), out, *ref):
         check_fp32(from_dev(got), r64, r32, name)
+
+
+# one block, several with a last one partly filled, exactly two cells per thread, and the
+# loop past the two cells a thread requests ahead (more than 1024 blocks of 512 cells)
+@pytest.mark.parametrize("shape", [(6, 6, 6), (19, 23, 17), (32, 32, 64), (96, 96, 60)], ids=str)
+def test_bicgstab_first_iterations_against_oracle(shape):
+    """Four BiCGSTAB iterations against the FP64 oracle.  The first iterations do not yet
+    amplify rounding: the FP32 oracle is 1e-7 to 1e-6 off after them, and the bound is 8x its
+    error, as for the other operators."""
+    import torch
+    from lex_amd import _lib
+    from oracle import lex_oracle as o
+    from tests._helpers import check_fp32
+    nx, ny, nz = shape
+    gr = o.Grid(nx, ny, nz, 600.0, 600.0, 300.0)
+    rng = np.random.default_rng(11)
+    rtt = np.asarray(rng.uniform(200.0, 350.0, gr.shape_c), np.float32)
+    rtt[:, :, 0] = rtt[:, :, -1] = 0.0   # no buoyancy: the operator is linear
+    b = np.asarray(o.laplace_of_pressure(rtt.astype(np.float64), rng.normal(0, 1e-3, shape), gr), np.float32)
+    x0 = np.asarray(rng.normal(0, 1e-4, shape), np.float32)
+    ref = [o.bicgstab(lambda x, dt=dt: o.laplace_of_pressure(rtt.astype(dt), x, gr), b.astype(dt), x0.astype(dt), 1e-12,
+                      0.0, 4) for dt in (np.float64, np.float32)]
+    g = _lib.grid(nx, ny, nz, gr.dx, gr.dy, gr.dz)
+    ws = torch.empty(_lib.load().lex_bicgstab_workspace_bytes(g), dtype=torch.uint8, device="cuda")
+    rt, bd, xd = to_dev(rtt), to_dev(b), to_dev(x0)
+    x = torch.empty_like(xd)
+    import ctypes
+    k = ctypes.c_int(-99)
+    _lib.call("lex_bicgstab", g, _lib.ptr(rt), _lib.ptr(bd), _lib.ptr(xd), _lib.ptr(x), 1e-12, 0.0, 4, _lib.ptr(ws),
+              ws.numel(), ctypes.byref(k), _lib.stream())
+    assert k.value == ref[0][1] == 4
+    check_fp32(from_dev(x), ref[0][0], ref[1][0], "x")
