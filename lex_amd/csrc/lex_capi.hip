@@ -1084,38 +1084,29 @@ namespace {
 template <int CI, int CO>
 void launch_fwd(int nx, int ny, int nz, const void* x, const void* wp, const float* bias, int mode, int cout_real,
                 void* y, float* yf, float* pre, hipStream_t st) {
-  if (CI <= 32 && CO == 32) {   // persistent, weights in registers
-    constexpr int CIP = CI <= 32 ? CI : 32;
-#define LEX_FWD32P(MD)                                                                                  \
-  if ((mode & 15) == MD) {                                                                               \
-    hipLaunchKernelGGL((k_conv3_fwd32p<CIP, MD>), dim3(conv_fwd32p_grid<CIP, MD>(nx, ny, nz)), dim3(256), 0, st, \
-                       nx, ny, nz, (const __bf16*)x, (const __bf16*)wp, bias, cout_real, (__bf16*)y, yf, pre); \
-    return;                                                                                             \
+  if constexpr (CI <= 32 && CO <= 32) {   // weights in registers, march along x
+    const int tz = (nz + RTZ - 1) / RTZ, ty = (ny + RTY - 1) / RTY;
+#define LEX_ROWS(MD)                                                                                          \
+  if ((mode & 15) == MD) {                                                                                    \
+    const int run = conv_run(nx, tz * ty, conv_rows_resident<CI, CO, MD>());                                  \
+    hipLaunchKernelGGL((k_conv3_rows<CI, CO, MD>), dim3(tz, ty, (nx + run - 1) / run), dim3(256), 0, st, nx, ny, nz, \
+                       run, (const __bf16*)x, (const __bf16*)wp, bias, cout_real, (__bf16*)y, yf, pre);        \
+    return;                                                                                                   \
   }
-    LEX_FWD32P(0) LEX_FWD32P(1) LEX_FWD32P(2) LEX_FWD32P(3) LEX_FWD32P(4) LEX_FWD32P(5) LEX_FWD32P(6) LEX_FWD32P(7)
-    LEX_FWD32P(8)
-#undef LEX_FWD32P
-  }
-  if (CO % 32 == 0) {   // 32 x 32 MFMA tiles: one A fragment per 32 output channels
+    LEX_ROWS(0) LEX_ROWS(1) LEX_ROWS(2) LEX_ROWS(3) LEX_ROWS(4) LEX_ROWS(5) LEX_ROWS(6) LEX_ROWS(7)
+    if constexpr (CO == 32) {
+      LEX_ROWS(8)
+    }
+#undef LEX_ROWS
+  } else if constexpr (CO % 32 == 0) {   // 32 x 32 MFMA tiles: one A fragment per 32 output channels
     dim3 grid((nz + CT2Z - 1) / CT2Z, (ny + CT2Y - 1) / CT2Y, (nx + CT2X - 1) / CT2X);
-    hipLaunchKernelGGL((k_conv3_fwd32<CI, (CO % 32 == 0 ? CO : 32)>), grid, dim3(256), 0, st, nx, ny, nz,
-                       (const __bf16*)x, (const __bf16*)wp, bias, mode, cout_real, (__bf16*)y, yf, pre);
-    return;
+    hipLaunchKernelGGL((k_conv3_fwd32<CI, CO>), grid, dim3(256), 0, st, nx, ny, nz, (const __bf16*)x, (const __bf16*)wp,
+                       bias, mode, cout_real, (__bf16*)y, yf, pre);
+  } else {
+    dim3 grid((nz + CTZ - 1) / CTZ, (ny + CTY - 1) / CTY, (nx + CTX - 1) / CTX);
+    hipLaunchKernelGGL((k_conv3_fwd<CI, CO>), grid, dim3(256), 0, st, nx, ny, nz, (const __bf16*)x, (const __bf16*)wp,
+                       bias, mode, cout_real, (__bf16*)y, yf, pre);
   }
-  if (CI <= 32 && CO == 16) {   // persistent, weights in registers
-    constexpr int CIP = CI <= 32 ? CI : 32;
-#define LEX_FWDP(MD)                                                                                   \
-  if ((mode & 7) == MD) {                                                                              \
-    hipLaunchKernelGGL((k_conv3_fwdp<CIP, MD>), dim3(conv_fwdp_grid<CIP, MD>(nx, ny, nz)), dim3(256), 0, st, \
-                       nx, ny, nz, (const __bf16*)x, (const __bf16*)wp, bias, cout_real, (__bf16*)y, yf, pre); \
-    return;                                                                                            \
-  }
-    LEX_FWDP(0) LEX_FWDP(1) LEX_FWDP(2) LEX_FWDP(3) LEX_FWDP(4) LEX_FWDP(5) LEX_FWDP(6) LEX_FWDP(7)
-#undef LEX_FWDP
-  }
-  dim3 grid((nz + CTZ - 1) / CTZ, (ny + CTY - 1) / CTY, (nx + CTX - 1) / CTX);
-  hipLaunchKernelGGL((k_conv3_fwd<CI, CO>), grid, dim3(256), 0, st, nx, ny, nz, (const __bf16*)x, (const __bf16*)wp,
-                     bias, mode, cout_real, (__bf16*)y, yf, pre);
 }
 // workgroups of k_conv3_wgrad: one per CU (the accumulators fill the register file)
 inline unsigned wgrad_blocks(int nx, int ny, int nz) {
@@ -1143,7 +1134,7 @@ static int conv_fwd(const char* name, int nx, int ny, int nz, int cin, int cout,
   if ((mode & 2) ? !yf : !y) return fail(-2, "%s: missing output", name);
   if ((mode & 4) && (nx < 2 || ny < 2)) return fail(-1, "%s: periodic padding needs nx, ny >= 2", name);
   const int cip = padc(cin), cop = padc(cout);
-  // the GELU-gradient epilogue (mode 8) exists in the persistent 32-output-channel kernel only
+  // the GELU-gradient epilogue (mode 8) exists for 32 output channels in the marching kernel only
   if ((mode & 8) && (mode != 8 || cip > 32 || cop != 32 || !pre))
     return fail(-1, "%s: the fused GELU gradient needs <= 32 input and 17..32 output channels", name);
 #define LEX_FWD(CI, CO) \

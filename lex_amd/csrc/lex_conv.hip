@@ -18,6 +18,7 @@
 namespace lex {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int CTX = 4, CTY = 4, CTZ = 16;  // output tile of one workgroup (4 waves)
@@ -266,358 +267,257 @@ __global__ __launch_bounds__(256) void k_conv3_fwd32(int nx, int ny, int nz, con
   }
 }
 
-// Persistent form for CIN <= 32 and 32 output channels (the SGS net's 32-channel layers).
-// Workgroup b owns the contiguous tile range [b T / G, (b+1) T / G) (z tiles fastest, then
-// y, then x): consecutive tiles of one workgroup share halo cells in its L2.  The weight
-// fragments of every K step stay in registers for the whole launch (NK x 4 VGPRs: 216 for
-// 32 input channels, so one wave per SIMD; 108 for 16, which fit two), the halo of tile
-// t+1 is fetched into registers while tile t's MFMAs and epilogue run, and the K loop
-// reads only LDS.  MODE: bit 0 GELU after the bias, bit 1 FP32 output Yf with cout_real
-// channels (else BF16 Y), bit 2 periodic x and y, bit 3 GELU gradient: `pre` is read (the
-// FP32 pre-activation of the layer below, 32 channels) and Y = BF16((acc + bias) *
-// gelu'(pre)), the data gradient and the k_gelu_bwd pass after it in one (bits 0-2
-// clear).  Same results as k_conv3_fwd32 (and, bit 3, as that pair).
-template <int CIN, int MODE>
-__global__ __launch_bounds__(256, CIN <= 16 ? 2 : 1) void k_conv3_fwd32p(int nx, int ny, int nz, const __bf16* __restrict__ X,
-                                                      const __bf16* __restrict__ Wp, const float* __restrict__ bias,
-                                                      int cout_real, __bf16* __restrict__ Y, float* __restrict__ Yf,
-                                                      float* __restrict__ pre) {
-  constexpr int COUT = 32;
-  static_assert(CIN <= 32, "persistent form: the weights of CIN <= 32 fit the register file");
-  constexpr int NSTEP = ConvSteps<CIN>::NSTEP, NK = 2 * NSTEP;   // 16-wide K steps
-  constexpr int GX = CT2X + 2, GY = CT2Y + 2, GZ = CT2Z + 2, CS = conv_cell_stride(CIN);
-  constexpr int NCH = CIN / 8, NTOT = GX * GY * GZ * NCH, NPF = (NTOT + 255) / 256;  // 16-byte chunks
+// The forward convolution for CIN <= 32 and 16 or 32 output channels (every layer of the SGS
+// net and simpleCNN, both directions): a march along x with the weights in registers.
+//
+// A workgroup of 4 waves owns a column of 4 y rows and 16 z cells and a run of x planes, which
+// it advances 4 at a time.  A wave owns 16 output channels (the MFMA's rows) and, of the four
+// planes, WX (2 with 32 output channels, where two waves share a plane, 1 with 16) of 4 y rows
+// of 16 z cells (the MFMA's columns).  An operand read from LDS (16 cells of one z run x 32 k)
+// is used for every (x, y) tap that reaches it: 3 (WX 2) or 2 MFMAs per read on average; one
+// per read, as with the cells as rows of one plane, needs all the LDS bandwidth there is.
+// Half the output channels per wave is half the weights (108 VGPRs for 32 input channels),
+// which leaves two waves per SIMD.
+//
+// LDS is a ring of 10 halo planes (6 rows x 18 cells): 6 that the step reads and the next 4,
+// which arrive straight from memory (no registers) under the step's MFMAs.  The results are
+// stored after the wait for them, so that no wait covers a store just issued.  The march
+// reads each x plane once (108 cells per 64 outputs; a stand-alone 8 x 4 x 16 tile 135), and
+// neighbouring columns, on one XCD, read their common rows at about the same time.
+//
+// Neither unit is saturated: at 240 x 240 x 120 the 32 -> 32 layer takes 366 us, its MFMAs
+// alone 240 (a third of them 112, so 192 for the MFMAs themselves, 2.0 GHz under that load)
+// and its memory traffic alone (0.52 GB read, 0.43 written) 215.  One wave per SIMD with all
+// the weights, 4 x 4 x 16 tiles and 32 x 32 MFMAs took 575 there and 42 (now 31) at 96 x 96 x
+// 48; 5 -> 32 277 (now 236) and 32 -> 5 287 (220).  No gain from wave priorities, from
+// non-temporal stores (pre-activations 20 % slower) or from three waves per SIMD for 16
+// input channels (365 us: spills).
+//
+// K: for 32 input channels one step per tap; for 16 a step is two z taps, (-1, 0) and (+1, -),
+// lanes 0-31 reading the first and 32-63 the second.  Cells lie unpadded in LDS; for 32
+// channels the upper and lower 32 bytes of a cell change places where bit 2 of its z position
+// is set, which puts the 16 lanes that an operand read serves at a time (0-3, 12-15, 20-27 and
+// 4-11, 16-19, 28-31 of each half wave) on all 64 banks.
+//
+// MODE: bit 0 GELU after the bias, bit 1 FP32 output Yf with cout_real channels (else BF16
+// Y), bit 2 periodic x and y, bit 3 GELU gradient: `pre` is read (the FP32 pre-activation of
+// the layer below, COUT channels) and Y = BF16((acc + bias) * gelu'(pre)), the data gradient
+// and the k_gelu_bwd pass after it in one (bits 0-2 clear).
+constexpr int RSX = 4, RTY = 4, RTZ = 16;   // planes per step; rows and cells of a column
+constexpr int RRING = 2 * RSX + 2;          // halo planes in LDS
+
+__device__ const unsigned k_zero_chunk[4] __attribute__((aligned(16))) = {0, 0, 0, 0};
+
+template <int CIN, int COUT, int MODE>
+__global__ __launch_bounds__(256, 2) void k_conv3_rows(int nx, int ny, int nz, int run, const __bf16* __restrict__ X,
+                                                       const __bf16* __restrict__ Wp, const float* __restrict__ bias,
+                                                       int cout_real, __bf16* __restrict__ Y, float* __restrict__ Yf,
+                                                       float* __restrict__ pre) {
+  static_assert((CIN == 16 || CIN == 32) && (COUT == 16 || COUT == 32), "weights and accumulators fit 256 VGPRs");
   constexpr bool GELU = (MODE & 1) != 0, F32 = (MODE & 2) != 0, CIRC = (MODE & 4) != 0, GGRAD = (MODE & 8) != 0;
   static_assert(!GGRAD || (MODE & 7) == 0, "the GELU-gradient epilogue writes BF16 without GELU");
-  constexpr bool PF = GGRAD && CIN > 16;   // pre-activations prefetched for the whole tile
-  // LDS row (one z run of GZ cells) stride RS elements, padded to 256 bytes modulo 512: an
-  // operand read takes two z runs of 16 cells in adjacent rows (lanes 0-15, 16-31), whose
-  // 16-byte slots then fall on the two complementary halves of the 512-byte bank row
-  constexpr int RS = (GZ * CS * 2 + (((256 - GZ * CS * 2) % 512) + 512) % 512) / 2;
-  static_assert((RS * 2) % 512 == 256, "row stride");
-  __shared__ __attribute__((aligned(16))) __bf16 tile[GX * GY * RS];
-  const int ntz = (nz + CT2Z - 1) / CT2Z, nty = (ny + CT2Y - 1) / CT2Y, ntx = (nx + CT2X - 1) / CT2X;
-  const int ntiles = ntz * nty * ntx;
-  const int t_begin = (int)((long)blockIdx.x * ntiles / gridDim.x);
-  const int t_end = (int)((long)(blockIdx.x + 1) * ntiles / gridDim.x);
-  if (t_begin >= t_end) return;  // uniform over the workgroup
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, m = l & 31, h = l >> 5;
-  const float bn = bias[m];
-  bf16x8 wr[NK];
+  constexpr int NH = COUT / 16, WX = NH;                        // channel halves; planes per wave and step
+  constexpr int GY = RTY + 2, GZ = RTZ + 2, NCH = CIN / 8;      // halo rows, cells; 16-byte chunks of a cell
+  constexpr int PLC = GY * GZ * NCH, GP = (PLC + 63) / 64;      // chunks of a plane; wave accesses that fetch it
+  constexpr int PLANE = GP * 64 * 8;                            // LDS elements of a plane
+  constexpr int NPF = (RSX * GP + 3) / 4;                       // accesses per wave and step
+  constexpr int NZG = CIN == 32 ? 3 : 2;                        // K steps per (x, y) tap
+  constexpr int KROW = ConvSteps<CIN>::NSTEP * 32;              // packed weights of one output channel
+  __shared__ __attribute__((aligned(16))) __bf16 ring[RRING * PLANE];
+  const TileId tb = xcd_tile();
+  const int z0 = tb.x * RTZ, y0 = tb.y * RTY, xa = tb.z * run, xb = min(xa + run, nx);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, m = l & 15, g = l >> 4;
+  const int ch = (w % NH) * 16 + 4 * g, xw = (w / NH) * WX;     // first output channel of the lane; first plane
+  auto swz = [](int z) { return CIN == 32 ? (z >> 1) & 2 : 0; };
+  // weights: rows are output channels, k this lane's 8 channels of the step's tap (CIN 16:
+  // tap slot 27 of the packed rows is zero)
+  bf16x8 wr[9][NZG];
   {
-    const __bf16* wl = Wp + (long)m * (NSTEP * 32) + 8 * h;
+    const __bf16* wl = Wp + (long)((w % NH) * 16 + m) * KROW + 8 * (g % NCH);
 #pragma unroll
-    for (int s = 0; s < NK; ++s) wr[s] = *(const bf16x8*)(wl + s * 16);
+    for (int xy = 0; xy < 9; ++xy)
+#pragma unroll
+      for (int zg = 0; zg < NZG; ++zg) {
+        const int tap = CIN == 32 ? xy * 3 + zg : (zg == 0 ? xy * 3 + (g >> 1) : (g < 2 ? xy * 3 + 2 : 27));
+        wr[xy][zg] = *(const bf16x8*)(wl + tap * CIN);
+      }
   }
-  bf16x8 pf[NPF];
-  // thread t loads chunk t % NCH of halo cells t / NCH + STEP j; the cell coordinates
-  // advance by a constant per j (no divisions per tile)
-  constexpr int STEP = 256 / NCH, SZ = STEP % GZ, SY = (STEP / GZ) % GY, SX = STEP / (GZ * GY);
-  const int g = threadIdx.x % NCH, q0 = threadIdx.x / NCH;
-  const int hz0 = q0 % GZ, hy0 = (q0 / GZ) % GY, hx0 = q0 / (GZ * GY);
-  auto fetch = [&](int t) {
-    const int z0 = (t % ntz) * CT2Z, y0 = ((t / ntz) % nty) * CT2Y, x0 = (t / (ntz * nty)) * CT2X;
-    int hz = hz0, hy = hy0, hx = hx0;
+  const f32x4 bn = {bias[ch], bias[ch + 1], bias[ch + 2], bias[ch + 3]};
+  // LDS element of this lane's operand in step zg of row 0 of a plane
+  int lb[NZG];
 #pragma unroll
-    for (int j = 0; j < NPF; ++j) {
-      const int c = threadIdx.x + 256 * j;
-      bf16x8 v;
-      for (int e = 0; e < 8; ++e) v[e] = (__bf16)0.0f;
-      if (c < NTOT) {
-        int gx = x0 + hx - 1, gy = y0 + hy - 1;
-        const int gz = z0 + hz - 1;
+  for (int zg = 0; zg < NZG; ++zg) {
+    const int z = m + (CIN == 32 ? zg : (zg == 0 ? (g >> 1) : 2));
+    lb[zg] = z * CIN + 8 * ((g % NCH) ^ swz(z));
+  }
+  // Fetch access q of a run of planes: 64 consecutive chunks q % GP of plane q / GP.  The
+  // lane's chunk: row hy, cell hz, source chunk of the cell.
+  auto chunk = [&](int q, int& hy, int& hz) {
+    const int c = (q % GP) * 64 + l, cell = c / NCH;
+    hy = cell / GZ;
+    hz = cell - hy * GZ;
+    return 8 * ((c % NCH) ^ swz(hz));
+  };
+  auto put = [&](int q, int slot, const void* src) {
+    if (PLC % 64 == 0 || (q % GP) * 64 + l < PLC)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                       (__attribute__((address_space(3))) void*)(ring + slot * PLANE + (q % GP) * 512), 16, 0, 0);
+  };
+  // byte offsets of the lane's chunks of a step's planes from (plane, y0 - 1, z0 - 1)
+  uint32_t off[NPF];
+#pragma unroll
+  for (int j = 0; j < NPF; ++j) {
+    const int q = w + 4 * j;
+    int hy, hz;
+    const int e = chunk(q, hy, hz);
+    off[j] = (uint32_t)(((q / GP) * ny + hy) * nz + hz) * (CIN * 2) + 2 * e;
+  }
+  const bool inside = y0 > 0 && z0 > 0 && y0 + RTY < ny && z0 + RTZ < nz && (long)RRING * ny * nz * CIN * 2 < (1L << 32);
+  // n planes from x = px on (cells outside the domain: zero, or their periodic image) into
+  // the ring slots from `slot` on
+  auto fetch = [&](int px, int n, int slot) {
+    if (inside && n == RSX && px >= 0 && px + RSX <= nx) {   // uniform
+      const char* corner = (const char*)(X + (((long)px * ny + (y0 - 1)) * nz + (z0 - 1)) * CIN);
+#pragma unroll
+      for (int j = 0; j < NPF; ++j) {
+        const int q = w + 4 * j, s = slot + q / GP;
+        if ((RSX * GP) % 4 == 0 || q < RSX * GP) put(q, s >= RRING ? s - RRING : s, corner + (size_t)off[j]);
+      }
+    } else {
+      for (int q = w; q < n * GP; q += 4) {
+        int hy, hz;
+        const int e = chunk(q, hy, hz);
+        int gx = px + q / GP, gy = y0 + hy - 1;
+        const int gz = z0 + hz - 1, s = slot + q / GP;
         if (CIRC) {
           gx = gx < 0 ? gx + nx : (gx >= nx ? gx - nx : gx);
           gy = gy < 0 ? gy + ny : (gy >= ny ? gy - ny : gy);
         }
-        if ((unsigned)gx < (unsigned)nx && (unsigned)gy < (unsigned)ny && (unsigned)gz < (unsigned)nz)
-          v = *(const bf16x8*)(X + (((long)gx * ny + gy) * nz + gz) * CIN + 8 * g);
+        const void* src = X + (((long)gx * ny + gy) * nz + gz) * CIN + e;
+        if (!((unsigned)gx < (unsigned)nx && (unsigned)gy < (unsigned)ny && (unsigned)gz < (unsigned)nz)) src = k_zero_chunk;
+        put(q, s >= RRING ? s - RRING : s, src);
       }
-      pf[j] = v;
-      hz += SZ;
-      const int cz = hz >= GZ;
-      hz -= cz ? GZ : 0;
-      hy += SY + cz;
-      const int cy = hy >= GY;
-      hy -= cy ? GY : 0;
-      hx += SX + cy;
     }
   };
-  // LDS element offset of this thread's chunk j: cell (hx, hy, hz) at (hx GY + hy) RS + hz CS
-  auto lds_off = [&](int j) {
-    const int cell = q0 + STEP * j;
-    return ((cell / GZ) * RS + (cell % GZ) * CS) + 8 * g;   // constant-folded per j
-  };
-  fetch(t_begin);
-  // LDS operand of K step s for accumulator block mt: cell ((w + 1 + dx), (2 mt + m/16 +
-  // 1 + dy), (m%16 + 1 + dz)), channel ch0 + 8 h; the tap of a step is lane-independent
-  // base at the tap (-1, -1, -1) corner, so every offset below is a non-negative constant
-  // (an LDS instruction's immediate offset is unsigned)
-  const __bf16* tw = tile + (w * GY + (m >> 4)) * RS + (m & 15) * CS + 8 * h;
-  auto a_at = [&](int s, int mt) {
-    int tap, ch0;
-    conv_step_k(CIN, (s * 16) / 32, (s * 16) % 32, tap, ch0);
-    if (tap > 26) tap = 26;          // padded K: weights are zero there
-    const int ox = tap / 9, oy = (tap / 3) % 3, oz = tap % 3;
-    return *(const bf16x8*)(tw + (ox * GY + 2 * mt + oy) * RS + oz * CS + ch0);
-  };
-  constexpr int AD = 2;   // LDS operands fetched AD steps ahead
-  for (int t = t_begin; t < t_end; ++t) {
-    __syncthreads();  // every wave has finished reading the previous tile
+  fetch(xa - 1, RSX + 2, 0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int zc = z0 + m;
+  int slot = 0;   // ring slot of plane x - 1
+  for (int x = xa; x < xb; x += RSX) {
+    __syncthreads();   // the step's planes are in LDS, and the slots of the next are no longer read
+    if (x + RSX < xb) fetch(x + RSX + 1, RSX, slot + RSX + 2 >= RRING ? slot + RSX + 2 - RRING : slot + RSX + 2);
+    f32x4 acc[WX][RTY];
 #pragma unroll
-    for (int j = 0; j < NPF; ++j) {
-      const int c = threadIdx.x + 256 * j;
-      if (c < NTOT) *(bf16x8*)(tile + lds_off(j)) = pf[j];
+    for (int a = 0; a < WX; ++a)
+#pragma unroll
+      for (int b = 0; b < RTY; ++b) acc[a][b] = bn;
+    // operand groups (halo plane, step), one group of GY rows read ahead
+    constexpr int NG = NZG * (WX + 2);
+    bf16x8 f[2][GY];
+    auto read = [&](int gi, bf16x8(&d)[GY]) {
+      const int s = slot + xw + gi / NZG;
+      const __bf16* r = ring + (s >= RRING ? s - RRING : s) * PLANE + lb[gi % NZG];
+#pragma unroll
+      for (int y = 0; y < GY; ++y) d[y] = *(const bf16x8*)(r + y * GZ * CIN);
+    };
+    read(0, f[0]);
+#pragma unroll
+    for (int gi = 0; gi < NG; ++gi) {
+      if (gi + 1 < NG) read(gi + 1, f[(gi + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);  // the reads ahead of this group's MFMAs, not after them
+      const int xp = gi / NZG, zg = gi % NZG;
+#pragma unroll
+      for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
+        for (int kx = 0; kx < 3; ++kx) {
+          if (xp - kx < 0 || xp - kx >= WX) continue;
+#pragma unroll
+          for (int y = 0; y < RTY; ++y)
+            acc[xp - kx][y] = mfma16(wr[kx * 3 + ky][zg], f[gi & 1][y + ky], acc[xp - kx][y]);
+        }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
-    // GELU gradient: the tile's pre-activations, loaded ahead of the next tile's halo so
-    // that they arrive during the MFMAs and waiting for them does not wait for the halo
-    // (CIN <= 16, two waves per SIMD: no registers to spare, loaded per row below)
-    float pv[PF ? CT2Y / 2 : 1][2][8];
-    if constexpr (PF) {
-      const int z0 = (t % ntz) * CT2Z, y0 = ((t / ntz) % nty) * CT2Y, x0 = (t / (ntz * nty)) * CT2X;
-      const int xc = x0 + w;
+    slot = slot + RSX >= RRING ? slot + RSX - RRING : slot + RSX;
+    // epilogue: accumulator i of (a, b) is cell (x + xw + a, y0 + b, z0 + m), channel ch + i
+    auto rows = [&](auto&& f) {
 #pragma unroll
-      for (int mt = 0; mt < CT2Y / 2; ++mt)
+      for (int a = 0; a < WX; ++a) {
+        const int xc = x + xw + a;
+        if (xc >= xb) continue;  // uniform over the wave
 #pragma unroll
-        for (int yq = 0; yq < 2; ++yq)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const int yc = y0 + 2 * mt + yq, zc = z0 + 4 * h + 8 * (j / 4) + (j % 4);
-            pv[mt][yq][j] = (xc < nx && yc < ny && zc < nz) ? pre[(((long)xc * ny + yc) * nz + zc) * COUT + m] : 0.f;
-          }
-    }
-    if (t + 1 < t_end) fetch(t + 1);  // in flight during this tile's MFMAs and epilogue
-    f32x16 acc[CT2Y / 2];
-#pragma unroll
-    for (int a = 0; a < CT2Y / 2; ++a)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][i] = 0.f;
-    bf16x8 aq[AD][CT2Y / 2];
-#pragma unroll
-    for (int s = 0; s < AD; ++s)
-#pragma unroll
-      for (int mt = 0; mt < CT2Y / 2; ++mt) aq[s][mt] = a_at(s < NK ? s : NK - 1, mt);
-#pragma unroll
-    for (int s = 0; s < NK; ++s) {
-      bf16x8 a[CT2Y / 2];
-#pragma unroll
-      for (int mt = 0; mt < CT2Y / 2; ++mt) a[mt] = aq[s % AD][mt];
-      if (s + AD < NK) {
-#pragma unroll
-        for (int mt = 0; mt < CT2Y / 2; ++mt) aq[s % AD][mt] = a_at(s + AD, mt);
-      }
-#pragma unroll
-      for (int mt = 0; mt < CT2Y / 2; ++mt)
-        acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[mt], wr[s], acc[mt], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);  // keep the LDS prefetch distance written here
-    }
-    // epilogue: accumulator i of block mt is cell (x0 + w, y0 + 2 mt + i / 8, z0 + 4 h +
-    // zo), zo = 8 ((i / 4) % 2) + i % 4, output channel m; each (x, y) row is addressed
-    // from one base with constant offsets
-    const int z0 = (t % ntz) * CT2Z, y0 = ((t / ntz) % nty) * CT2Y, x0 = (t / (ntz * nty)) * CT2X;
-    const int xc = x0 + w;
-    const bool zfull = z0 + CT2Z <= nz;
-    if (xc < nx) {
-#pragma unroll
-      for (int mt = 0; mt < CT2Y / 2; ++mt) {
-#pragma unroll
-        for (int yq = 0; yq < 2; ++yq) {
-          const int yc = y0 + 2 * mt + yq;
-          if (yc >= ny) continue;  // uniform over the wave
-          const long c0 = ((long)xc * ny + yc) * nz + z0 + 4 * h;
-          float* pr = pre ? pre + c0 * COUT + m : nullptr;
-          float prow[8];   // GELU gradient without the tile prefetch: this row's 8 values first
-          if constexpr (GGRAD && !PF) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-              prow[j] = (z0 + 4 * h + 8 * (j / 4) + (j % 4) < nz) ? pr[(8 * (j / 4) + (j % 4)) * COUT] : 0.f;
-          }
-          auto out = [&](int j) {
-            const int zo = 8 * (j / 4) + (j % 4);
-            float v = acc[mt][8 * yq + j] + bn;
-            if constexpr (GGRAD) {
-              const float pa = PF ? pv[PF ? mt : 0][yq][j] : prow[j];
-              v = m < cout_real ? v * gelu_t_grad(pa) : 0.f;   // padded channels: +0
-            } else if (pr) {
-              pr[zo * COUT] = v;
-            }
-            if (GELU) v = gelu_t(v);
-            if (F32) {
-              if (m < cout_real) Yf[(c0 + zo) * cout_real + m] = v;
-            } else {
-              Y[(c0 + zo) * COUT + m] = (__bf16)v;
-            }
-          };
-          if (zfull) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) out(j);
-          } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-              if (z0 + 4 * h + 8 * (j / 4) + (j % 4) < nz) out(j);
-          }
+        for (int b = 0; b < RTY; ++b) {
+          if (y0 + b >= ny) continue;  // uniform
+          if (zc < nz) f(a, b, ((long)xc * ny + y0 + b) * nz + zc);
         }
       }
+    };
+    bf16x4 res[WX][RTY];
+    if constexpr (GGRAD) {
+      rows([&](int a, int b, long c0) {
+        const f32x4 pa = *(const f32x4*)(pre + c0 * COUT + ch);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)   // padded channels: +0
+          res[a][b][i] = (__bf16)(ch + i < cout_real ? acc[a][b][i] * gelu_t_grad(pa[i]) : 0.f);
+      });
+    } else if constexpr (!F32) {
+#pragma unroll
+      for (int a = 0; a < WX; ++a)
+#pragma unroll
+        for (int b = 0; b < RTY; ++b)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) res[a][b][i] = (__bf16)(GELU ? gelu_t(acc[a][b][i]) : acc[a][b][i]);
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's part of the next planes
+    rows([&](int a, int b, long c0) {
+      const f32x4 v = acc[a][b];
+      if (!GGRAD && pre) *(f32x4*)(pre + c0 * COUT + ch) = v;
+      if constexpr (F32) {
+        float* o = Yf + c0 * cout_real + ch;
+        f32x4 r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = GELU ? gelu_t(v[i]) : v[i];
+        if (cout_real == COUT) {
+          *(f32x4*)o = r;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (ch + i < cout_real) o[i] = r[i];
+        }
+      } else {
+        *(bf16x4*)(Y + c0 * COUT + ch) = res[a][b];
+      }
+    });
   }
 }
 
-// Persistent form of k_conv3_fwd for CIN <= 32 and 16 output channels (the net's output
-// layer and the data gradient of its input layer), organised as k_conv3_fwd32p: a
-// contiguous tile range per workgroup, every K step's weight fragment in registers
-// (NSTEP x 4 VGPRs), the next tile's halo fetched during the current tile's MFMAs and
-// epilogue.  Same MFMA layout and results as k_conv3_fwd.
-template <int CIN, int MODE>
-__global__ __launch_bounds__(256, 2) void k_conv3_fwdp(int nx, int ny, int nz, const __bf16* __restrict__ X,
-                                                    const __bf16* __restrict__ Wp, const float* __restrict__ bias,
-                                                    int cout_real, __bf16* __restrict__ Y, float* __restrict__ Yf,
-                                                    float* __restrict__ pre) {
-  constexpr int COUT = 16;
-  static_assert(CIN <= 32, "persistent form: the weights of CIN <= 32 fit the register file");
-  constexpr int NSTEP = ConvSteps<CIN>::NSTEP, CS = conv_cell_stride(CIN);
-  constexpr int NCH = CIN / 8, NTOT = HX * HY * HZ * NCH, NPF = (NTOT + 255) / 256;  // 16-byte chunks
-  constexpr bool GELU = (MODE & 1) != 0, F32 = (MODE & 2) != 0, CIRC = (MODE & 4) != 0;
-  __shared__ __attribute__((aligned(16))) __bf16 tile[HX * HY * HZ * CS];
-  const int ntz = (nz + CTZ - 1) / CTZ, nty = (ny + CTY - 1) / CTY, ntx = (nx + CTX - 1) / CTX;
-  const int ntiles = ntz * nty * ntx;
-  const int t_begin = (int)((long)blockIdx.x * ntiles / gridDim.x);
-  const int t_end = (int)((long)(blockIdx.x + 1) * ntiles / gridDim.x);
-  if (t_begin >= t_end) return;  // uniform over the workgroup
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, m = l & 15, g = l >> 4;
-  const int kl = 8 * g;  // this lane's first k within a step
-  const float bn = bias[m];
-  bf16x8 wr[NSTEP];
-#pragma unroll
-  for (int s = 0; s < NSTEP; ++s) wr[s] = *(const bf16x8*)(Wp + (long)m * (NSTEP * 32) + s * 32 + kl);
-  constexpr int STEP = 256 / NCH, SZ = STEP % HZ, SY = (STEP / HZ) % HY, SX = STEP / (HZ * HY);
-  const int gc = threadIdx.x % NCH, q0 = threadIdx.x / NCH;
-  const int hz0 = q0 % HZ, hy0 = (q0 / HZ) % HY, hx0 = q0 / (HZ * HY);
-  bf16x8 pf[NPF];
-  auto fetch = [&](int t) {
-    const int z0 = (t % ntz) * CTZ, y0 = ((t / ntz) % nty) * CTY, x0 = (t / (ntz * nty)) * CTX;
-    int hz = hz0, hy = hy0, hx = hx0;
-#pragma unroll
-    for (int j = 0; j < NPF; ++j) {
-      const int c = threadIdx.x + 256 * j;
-      bf16x8 v;
-      for (int e = 0; e < 8; ++e) v[e] = (__bf16)0.0f;
-      if (c < NTOT) {
-        int gx = x0 + hx - 1, gy = y0 + hy - 1;
-        const int gz = z0 + hz - 1;
-        if (CIRC) {
-          gx = gx < 0 ? gx + nx : (gx >= nx ? gx - nx : gx);
-          gy = gy < 0 ? gy + ny : (gy >= ny ? gy - ny : gy);
-        }
-        if ((unsigned)gx < (unsigned)nx && (unsigned)gy < (unsigned)ny && (unsigned)gz < (unsigned)nz)
-          v = *(const bf16x8*)(X + (((long)gx * ny + gy) * nz + gz) * CIN + 8 * gc);
-      }
-      pf[j] = v;
-      hz += SZ;
-      const int cz = hz >= HZ;
-      hz -= cz ? HZ : 0;
-      hy += SY + cz;
-      const int cy = hy >= HY;
-      hy -= cy ? HY : 0;
-      hx += SX + cy;
-    }
-  };
-  fetch(t_begin);
-  // LDS operand of step s for y row mt: cell (w + 1 + dx, mt + 1 + dy, m + 1 + dz), channel
-  // ch0 (tap and channel of the lane's k group, conv_step_k)
-  // base at the tap (-1, -1, -1) corner: non-negative constant offsets when the tap of a
-  // step is lane-independent (CIN = 32)
-  const __bf16* tc = tile + ((w * HY) * HZ + m) * CS;
-  auto a_at = [&](int s, int mt) {
-    int tap, ch0;
-    conv_step_k(CIN, s, kl, tap, ch0);
-    if (tap > 26) tap = 26;              // padded K step: weights are zero there
-    const int ox = tap / 9, oy = (tap / 3) % 3, oz = tap % 3;
-    return *(const bf16x8*)(tc + ((ox * HY + mt + oy) * HZ + oz) * CS + ch0);
-  };
-  for (int t = t_begin; t < t_end; ++t) {
-    __syncthreads();  // every wave has finished reading the previous tile
-#pragma unroll
-    for (int j = 0; j < NPF; ++j) {
-      const int c = threadIdx.x + 256 * j;
-      if (c < NTOT) *(bf16x8*)(tile + (q0 + STEP * j) * CS + 8 * gc) = pf[j];
-    }
-    __syncthreads();
-    if (t + 1 < t_end) fetch(t + 1);  // in flight during this tile's MFMAs and epilogue
-    f32x4 acc[CTY];
-#pragma unroll
-    for (int a = 0; a < CTY; ++a) acc[a] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    bf16x8 an[CTY];
-#pragma unroll
-    for (int mt = 0; mt < CTY; ++mt) an[mt] = a_at(0, mt);
-#pragma unroll
-    for (int s = 0; s < NSTEP; ++s) {
-      bf16x8 a[CTY];
-#pragma unroll
-      for (int mt = 0; mt < CTY; ++mt) a[mt] = an[mt];
-      if (s + 1 < NSTEP) {
-#pragma unroll
-        for (int mt = 0; mt < CTY; ++mt) an[mt] = a_at(s + 1, mt);
-      }
-#pragma unroll
-      for (int mt = 0; mt < CTY; ++mt) acc[mt] = mfma16(a[mt], wr[s], acc[mt]);
-      __builtin_amdgcn_sched_barrier(0);  // keep the LDS prefetch distance written here
-    }
-    // epilogue: accumulator i of row mt is cell (x0 + w, y0 + mt, z0 + 4 g + i), channel m
-    const int z0 = (t % ntz) * CTZ, y0 = ((t / ntz) % nty) * CTY, x0 = (t / (ntz * nty)) * CTX;
-    const int xc = x0 + w;
-    if (xc < nx) {
-#pragma unroll
-      for (int mt = 0; mt < CTY; ++mt) {
-        const int yc = y0 + mt;
-        if (yc >= ny) continue;  // uniform over the wave
-        const long c0 = ((long)xc * ny + yc) * nz + z0 + 4 * g;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (z0 + 4 * g + i < nz) {
-            float v = acc[mt][i] + bn;
-            if (pre) pre[(c0 + i) * COUT + m] = v;
-            if (GELU) v = gelu_t(v);
-            if (F32) {
-              if (m < cout_real) Yf[(c0 + i) * cout_real + m] = v;
-            } else {
-              Y[(c0 + i) * COUT + m] = (__bf16)v;
-            }
-          }
-        }
-      }
+// x planes per workgroup: whole steps, so many that the workgroups fill the device evenly.
+// A run costs its planes and about one step more (the first planes, the weights).
+inline int conv_run(int nx, int cols, int resident) {
+  int best = 0;
+  double cost = 0.0;
+  for (int runs = 1; runs <= (nx + RSX - 1) / RSX && runs <= 256; ++runs) {
+    const int len = ((nx + runs - 1) / runs + RSX - 1) / RSX * RSX;
+    const long n = (long)cols * ((nx + len - 1) / len);
+    const double c = (double)((n + resident - 1) / resident) * (len + RSX);
+    if (best == 0 || c < cost) {
+      best = len;
+      cost = c;
     }
   }
+  return best;
 }
 
-template <int CIN, int MODE>
-inline unsigned conv_fwdp_grid(int nx, int ny, int nz) {
-  static int resident = 0;
-  if (resident == 0) {
+// workgroups the device holds at once (occupancy from the runtime)
+template <int CIN, int COUT, int MODE>
+inline int conv_rows_resident() {
+  static const int resident = [] {
     int dev = 0, ncu = 0, per = 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_conv3_fwdp<CIN, MODE>, 256, 0);
-    resident = (ncu > 0 ? ncu : 256) * (per > 0 ? per : 1);
-  }
-  const long ntiles = (long)((nz + CTZ - 1) / CTZ) * ((ny + CTY - 1) / CTY) * ((nx + CTX - 1) / CTX);
-  return (unsigned)(ntiles < resident ? ntiles : resident);
-}
-
-// persistent grid of k_conv3_fwd32p: as many workgroups as the device holds at once
-// (occupancy from the runtime), at most one per tile
-template <int CIN, int MODE>
-inline unsigned conv_fwd32p_grid(int nx, int ny, int nz) {
-  static int resident = 0;
-  if (resident == 0) {
-    int dev = 0, ncu = 0, per = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_conv3_fwd32p<CIN, MODE>, 256, 0);
-    resident = (ncu > 0 ? ncu : 256) * (per > 0 ? per : 1);
-  }
-  const long ntiles = (long)((nz + CT2Z - 1) / CT2Z) * ((ny + CT2Y - 1) / CT2Y) * ((nx + CT2X - 1) / CT2X);
-  return (unsigned)(ntiles < resident ? ntiles : resident);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_conv3_rows<CIN, COUT, MODE>, 256, 0);
+    return (ncu > 0 ? ncu : 256) * (per > 0 ? per : 1);
+  }();
+  return resident;
 }
 
 // Weight gradient: dW[tap][c][n] += sum_p X[p + o(tap)][c] * G[p][n] over the cells of

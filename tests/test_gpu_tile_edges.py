@@ -100,3 +100,31 @@ def test_bicgstab_first_iterations_against_oracle(shape):
               ws.numel(), ctypes.byref(k), _lib.stream())
     assert k.value == ref[0][1] == 4
     check_fp32(from_dev(x), ref[0][0], ref[1][0], "x")
+
+
+# runs shorter than a step, of one step, and long enough to go round the ring of planes; one
+# and several rows and z tiles with and without a remainder; 16 and 32 channels either side
+@pytest.mark.parametrize("circular", [False, True])
+@pytest.mark.parametrize("cin,cout", [(5, 32), (32, 32), (32, 5), (16, 16)])
+@pytest.mark.parametrize("shape", [(4, 4, 16), (7, 5, 17), (46, 9, 35), (97, 66, 33)], ids=str)
+def test_convolution_march(shape, cin, cout, circular):
+    """One convolution against torch conv3d in float64 on the same BF16 operands: FP32 sums of
+    27 cin products, 1e-5 as for the other sizes; the BF16 output is its rounding (2^-8)."""
+    import torch
+    from lex_amd import sgs_net as sn
+    gen = torch.Generator().manual_seed(cin + cout)
+    x = torch.randn(*shape, cin, generator=gen)
+    W = torch.randn(27, cin, cout, generator=gen) / np.sqrt(27 * cin)
+    b = 0.1 * torch.randn(cout, generator=gen)
+    xb = x.bfloat16().double().permute(3, 0, 1, 2)[None]
+    wb = W.bfloat16().double().view(3, 3, 3, cin, cout).permute(4, 3, 0, 1, 2)
+    if circular:
+        xb = torch.nn.functional.pad(torch.nn.functional.pad(xb, (0, 0, 1, 1, 1, 1), mode="circular"), (1, 1))
+    else:
+        xb = torch.nn.functional.pad(xb, (1,) * 6)
+    ref = torch.nn.functional.conv3d(xb, wb, b.double())[0].permute(1, 2, 3, 0)
+    xd = sn.to_bf16_channels_last(x.cuda())
+    yf, _ = sn.conv3d_fwd(xd, shape, W.cuda(), b.cuda(), gelu=False, out_fp32=True, circular=circular)
+    yb, pre = sn.conv3d_fwd(xd, shape, W.cuda(), b.cuda(), gelu=False, out_fp32=False, want_pre=True, circular=circular)
+    rel = lambda a: float((a.cpu().double().view(*shape, -1)[..., :cout] - ref).norm() / ref.norm())  # noqa: E731
+    assert rel(yf) < 1e-5 and rel(pre) < 1e-5 and rel(yb) < 2.0 ** -8
