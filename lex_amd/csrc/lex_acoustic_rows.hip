@@ -9,9 +9,8 @@
 // cell-per-thread form 77 % busy (29 loads per cell; here 10 for one level, 20 of 8 bytes
 // for two).
 //
-// The arithmetic is acoustic_cell's operation by operation (contraction off, fmaf where it
-// has one), so the result is bit for bit that of k_acoustic2 and of a cell-per-thread
-// evaluation.
+// Contraction is spelled out (fmaf) and otherwise off, in k_acoustic and in both substeps of
+// k_acoustic2, so the results do not depend on which of them computed a cell.
 #pragma once
 #include <algorithm>
 #include "lex_ops.hip"
@@ -360,6 +359,391 @@ inline void launch_acoustic(const Dims& d, const AcousticArgs& a, hipStream_t st
     launch_acoustic_v<2>(d, a, st);
   else
     launch_acoustic_v<1>(d, a, st);
+}
+
+// k_acoustic2: two consecutive substeps in one launch, bit for bit what two k_acoustic
+// launches give.  A workgroup of R rows (the outer two are halo rows) marches along x; a wave
+// owns the 64 V levels of one row, as in k_acoustic.  In step s it
+//   finishes the y and z faces of the second substep at cell s - 1 (the neighbour rows' new
+//   pi' of that position is in LDS, everything else in its registers),
+//   advances cell s by the first substep and puts the new pi' into LDS,
+//   asks for the operands of cell s + 1,
+//   finishes the second substep at cell s - 1, whose x face needed the new pi' of cell s,
+// with one barrier per step and two slabs of pi'.  Halo rows and the positions x0 - 1 and x1
+// are taken at their periodic images, so the second substep reads what it would read from
+// the ghosts.
+//
+// Bound by memory (the thirteen fields once for two substeps: 72 us at 240x240x120 and
+// 5 TB/s) and by the barrier that holds a CU's waves together.  us per pair against two
+// k_acoustic launches: 40x40x40 9.8 and 19, 96x96x48 19 and 23, 128x128x64 23 and 31,
+// 181x147x70 57 and 64, 192x160x96 65 and 76, 128x128x160 80 and 86, 240x240x120 142 and 198,
+// 256x256x128 152 and 228, 256x256x200 309 and 441, 512x512x64 337 and 438, so every pair of
+// substeps takes it.  With a cell per thread, faces evaluated twice and the levels exchanged
+// through the LDS pipe it took 194 and 194 at 240x240x120 and 256x256x128.  Eight rows of two
+// levels per lane: 166 and 188, sixteen (spills) 172 and 194.
+template <int V>
+struct Pair2Operands {
+  float p1[V], t1[V], s1[V];               // row j of plane x + 1
+  float py[2][V], ty[2][V], sy[2][V];      // rows j - 1, j + 1 of plane x
+  float uf[V], gu[V], vf[2][V], gv[2][V], wf[V], gw[V];
+  float pe, te, se, we, ge;                // beyond the wave's levels (edge lanes)
+};
+
+template <int V, bool MZ, int MAXT>
+__global__ void __launch_bounds__(MAXT) k_acoustic2(Dims d, AcousticArgs a, int ax) {
+#pragma clang fp contract(off)
+  extern __shared__ float ring[];  // [2 slabs][R rows][64 V levels of every wave of a row]
+  const int lane = threadIdx.x & 63;
+  const int chunk = MZ ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
+  const int r = __builtin_amdgcn_readfirstlane((int)threadIdx.y), R = blockDim.y, LR = blockDim.x * V;
+  const TileId tb = xcd_tile();
+  const int nx = d.nx, ny = d.ny, nz = d.nz;
+  const int j = tb.x * (R - 2) - 1 + r;          // -1 .. ny (rows past ny repeat it, never stored)
+  const int jw = wrap_cell(min(j, ny), ny);
+  const bool rowb = r >= 1 && r <= R - 2 && j < ny;
+  const int x0 = tb.y * ax, x1 = min(x0 + ax, nx);
+  const int kl = (chunk * 64 + lane) * V;
+  const int kc = min(kl, nz - 1);
+  LevelSlots ls;
+  ls.n = min(max(nz - kl, 0), V);
+  ls.first = kl == 0;
+  ls.last = ls.n > 0 && kl + ls.n == nz;
+  const uint32_t eK = (uint32_t)(kc + 1);
+  const uint32_t ek = (uint32_t)min(kc, nz - V);
+  const bool past = (V == 2) && kc == nz - 1;
+  const float h = (float)(-kCp * 0.5);
+  const float dts = a.dts;
+  float rr[V], ir[V], r8[V], pic[V], dpi[V];
+#pragma unroll
+  for (int q = 0; q < V; ++q) {
+    const int K = min(kc + q + 1, nz + 1);
+    rr[q] = a.rc[K];
+    ir[q] = 1.0f / rr[q];
+    r8[q] = 0.5f * (a.rc[K - 1] + rr[q]);
+    pic[q] = a.pi0[K];
+    dpi[q] = (pic[q] - a.pi0[K - 1]) * d.idz;
+  }
+  float r8e = 0.f, dpie = 0.f;
+  if (MZ) {
+    const int K = min(kc + V + 1, nz + 1);
+    r8e = 0.5f * (a.rc[K - 1] + a.rc[K]);
+    dpie = (a.pi0[K] - a.pi0[K - 1]) * d.idz;
+  }
+  const bool edge = MZ && (lane == 0 || lane == 63);
+  const uint32_t eE = (uint32_t)(lane == 0 ? kc : min(kc + V + 1, nz + 1));
+  const uint32_t eW = (uint32_t)min(kc + V, nz);
+
+  const int syc = nz + 2, syw = nz + 3;
+  const int sxc = (ny + 6) * syc, sxv = (ny + 7) * syc, sxw = (ny + 6) * syw;
+  const int sxiu = ny * nz, sxiv = (ny + 1) * nz, sxiw = ny * (nz + 1);
+  const uint32_t oc = (uint32_t)((jw + 3) * syc) + eK, ow = (uint32_t)((jw + 3) * syw) + eK;
+  const uint32_t ocm = oc - (uint32_t)syc, ocp = oc + (uint32_t)syc;
+  const uint32_t oi = (uint32_t)(jw * nz) + ek, oin = oi + (uint32_t)nz;
+  const uint32_t og = (uint32_t)(jw * (nz + 1) + kc);
+  float* const own = ring + r * LR + (chunk * 64 + lane) * V;
+  const int slab = R * LR;
+
+  // input planes of the cell in hand
+  const float *pX, *tX, *sX, *uX, *vX, *wX, *guX, *gvX, *gwX;
+  auto place = [&](int xw) {
+    pX = a.p + (long)(xw + 3) * sxc;
+    tX = a.tr + (long)(xw + 3) * sxc;
+    sX = a.ps + (long)(xw + 3) * sxc;
+    uX = a.u + (long)(xw + 3) * sxc;
+    vX = a.v + (long)(xw + 3) * sxv;
+    wX = a.w + (long)(xw + 3) * sxw;
+    guX = a.ru + (long)xw * sxiu;
+    gvX = a.rv + (long)xw * sxiv;
+    gwX = a.rw + (long)xw * sxiw;
+  };
+  auto fetch = [&](Pair2Operands<V>& o) {
+    ld_levels<V>(pX, ocm, o.py[0]);
+    ld_levels<V>(tX, ocm, o.ty[0]);
+    ld_levels<V>(sX, ocm, o.sy[0]);
+    ld_levels<V>(pX, ocp, o.py[1]);
+    ld_levels<V>(tX, ocp, o.ty[1]);
+    ld_levels<V>(sX, ocp, o.sy[1]);
+    ld_levels<V>(vX, oc, o.vf[0]);
+    ld_levels<V>(vX, ocp, o.vf[1]);
+    ld_levels_in<V>(gvX, oi, past, o.gv[0]);
+    ld_levels_in<V>(gvX, oin, past, o.gv[1]);
+    ld_levels<V>(wX, ow, o.wf);
+    ld_levels<V>(gwX, og, o.gw);
+    if (edge) {
+      o.pe = ld32(pX, oc - eK + eE);
+      o.te = ld32(tX, oc - eK + eE);
+      o.se = ld32(sX, oc - eK + eE);
+      o.we = ld32(wX, ow - eK + eW + 1u);
+      o.ge = ld32(gwX, og - (uint32_t)kc + eW);
+    }
+    ld_levels<V>(pX + sxc, oc, o.p1);
+    ld_levels<V>(tX + sxc, oc, o.t1);
+    ld_levels<V>(sX + sxc, oc, o.s1);
+    ld_levels<V>(uX + sxc, oc, o.uf);
+    ld_levels_in<V>(guX + sxiu, oi, past, o.gu);
+  };
+
+  // first substep, row j of the cell in hand, and its lower x face: new u, u dpi*/dx
+  float P0[V], T0[V], S0[V], ul[V], dl[V];
+  // second substep: operands of cell s - 1 and of the x face in hand, new pi' there, new u
+  // and u dpi*/dx of its lower x face
+  float hty[2][V], dsy[2][V], gvb[2][V], vb[2][V], htz[V], dzb[V], gwb[V], wb[V], pab[V], pb[V];
+  float ub[V], gub[V], htx[V], dsx[V], ulb[V], dlb[V];
+  float hte = 0.f, dze = 0.f, geb = 0.f, web = 0.f;
+#pragma unroll
+  for (int q = 0; q < V; ++q) {
+    pb[q] = ulb[q] = dlb[q] = pab[q] = 0.f;
+    ub[q] = gub[q] = htx[q] = dsx[q] = 0.f;
+  }
+  Pair2Operands<V> o;
+  place(wrap_cell(x0 - 1, nx));
+  fetch(o);
+#pragma unroll 1
+  for (int s = x0 - 1; s <= x1; ++s) {
+    const bool second = s > x0 && rowb;
+    // y and z faces of the second substep at cell s - 1
+    float dvn[V], hdv[V], dwn[V], zz[V];
+    if (second) {
+      const int x = s - 1;
+      const float* L = own + ((s - x0) & 1) * slab;
+      float vn[2][V], pm[V], pp[V];
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        pm[q] = L[q - LR];
+        pp[q] = L[q + LR];
+      }
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        vn[0][q] = fmaf(fmaf(hty[0][q], (pb[q] - pm[q]) * d.idy, gvb[0][q]), dts, vb[0][q]);
+        vn[1][q] = fmaf(fmaf(hty[1][q], (pp[q] - pb[q]) * d.idy, gvb[1][q]), dts, vb[1][q]);
+        dvn[q] = vn[1][q] - vn[0][q];
+        hdv[q] = 0.5f * (vn[1][q] * dsy[1][q] + vn[0][q] * dsy[0][q]);
+      }
+      float wn[V], a0[V], b0[V];
+      float pl0 = lane_below(pb[V - 1]);
+      float pu = 0.f;
+      if (MZ && lane == 0 && kl > 0) pl0 = L[-1];
+      if (MZ && lane == 63) pu = kl + V < LR ? L[V] : 0.f;
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        const float pl = q ? pb[0] : pl0;
+        const float wv = fmaf(htz[q] * ((pb[q] - pl) * d.idz) + gwb[q], dts, wb[q]);
+        const bool floor_ = q == 0 && kl == 0;
+        wn[q] = floor_ ? 0.0f : wv;
+        a0[q] = 0.5f * (floor_ ? 0.0f : wv * dzb[q]);
+        b0[q] = a0[q] * r8[q];
+      }
+      float wt = lane_above(wn[0]), bt = lane_above(b0[0]);
+      if (MZ && lane == 63) {
+        wt = fmaf(hte * ((pu - pb[V - 1]) * d.idz) + geb, dts, web);
+        bt = (0.5f * (wt * dze)) * r8e;
+      }
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        const bool lid = kl + q >= nz - 1;
+        const float w1 = lid ? 0.0f : (q < V - 1 ? wn[V - 1] : wt);
+        const float b1 = lid ? 0.0f : (q < V - 1 ? b0[V - 1] : bt);
+        dwn[q] = w1 - wn[q];
+        zz[q] = quotient(fmaf(a0[q], r8[q], b1), rr[q], ir[q]);
+      }
+      if (x >= 4 && x < nx - 3 && j >= 4 && j < ny - 3) {   // no periodic images
+        float* voX = a.vo + (long)(x + 3) * sxv;
+        float* woX = a.wo + (long)(x + 3) * sxw;
+        st_levels<V>(voX, oc, ls, vn[0]);
+        st_levels<V>(woX, ow, ls, wn);
+        if (ls.first || ls.last) {
+          st_ghosts<V>(voX, oc, ls, vn[0]);
+          st_ghosts_w<V>(woX, ow, ls, wn);
+        }
+      } else {
+        st_images<V, false>(a.vo, sxv, syc, x, nx, false, j, ny, true, eK, ls, vn[0]);
+        if (j == ny - 1) st_images<V, false>(a.vo, sxv, syc, x, nx, false, ny, ny, true, eK, ls, vn[1]);
+        st_images<V, true>(a.wo, sxw, syw, x, nx, false, j, ny, false, eK, ls, wn);
+      }
+    }
+    // a march starts, or continues at the other end of the period
+    if (s == x0 - 1 || s == 0 || s == nx) {
+      float pm[V], tm[V], sm[V], u0[V], g0[V];
+      ld_levels<V>(pX, oc, P0);
+      ld_levels<V>(tX, oc, T0);
+      ld_levels<V>(sX, oc, S0);
+      ld_levels<V>(pX - sxc, oc, pm);
+      ld_levels<V>(tX - sxc, oc, tm);
+      ld_levels<V>(sX - sxc, oc, sm);
+      ld_levels<V>(uX, oc, u0);
+      ld_levels_in<V>(guX, oi, past, g0);
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        const float ht = h * (T0[q] + tm[q]), ds = (S0[q] - sm[q]) * d.idx;
+        ul[q] = fmaf(fmaf(ht, (P0[q] - pm[q]) * d.idx, g0[q]), dts, u0[q]);
+        dl[q] = ul[q] * ds;
+        if (s <= x0) {   // the face where the second substep's march starts
+          ub[q] = ul[q];
+          gub[q] = g0[q];
+          htx[q] = ht;
+          dsx[q] = ds;
+        }
+      }
+    }
+    // first substep at cell s
+    float pn[V], pa1[V], ub1[V], gu1[V], htx1[V], dsx1[V];
+    {
+      float dv[2][V], div0[V];
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        hty[0][q] = h * (T0[q] + o.ty[0][q]);
+        hty[1][q] = h * (o.ty[1][q] + T0[q]);
+        dsy[0][q] = (S0[q] - o.sy[0][q]) * d.idy;
+        dsy[1][q] = (o.sy[1][q] - S0[q]) * d.idy;
+        vb[0][q] = fmaf(fmaf(hty[0][q], (P0[q] - o.py[0][q]) * d.idy, o.gv[0][q]), dts, o.vf[0][q]);
+        vb[1][q] = fmaf(fmaf(hty[1][q], (o.py[1][q] - P0[q]) * d.idy, o.gv[1][q]), dts, o.vf[1][q]);
+        gvb[0][q] = o.gv[0][q];
+        gvb[1][q] = o.gv[1][q];
+        dv[0][q] = vb[0][q] * dsy[0][q];
+        dv[1][q] = vb[1][q] * dsy[1][q];
+      }
+      float a0[V], b0[V];
+      float pl0 = lane_below(P0[V - 1]), tl0 = lane_below(T0[V - 1]), sl0 = lane_below(S0[V - 1]);
+      if (MZ && lane == 0) {
+        pl0 = o.pe;
+        tl0 = o.te;
+        sl0 = o.se;
+      }
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        const float pl = q ? P0[0] : pl0, tl = q ? T0[0] : tl0, sl = q ? S0[0] : sl0;
+        htz[q] = h * (T0[q] + tl);
+        dzb[q] = fmaf(S0[q] - sl, d.idz, dpi[q]);
+        gwb[q] = o.gw[q];
+        const float wv = fmaf(htz[q] * ((P0[q] - pl) * d.idz) + o.gw[q], dts, o.wf[q]);
+        const bool floor_ = q == 0 && kl == 0;
+        wb[q] = floor_ ? 0.0f : wv;
+        a0[q] = 0.5f * (floor_ ? 0.0f : wv * dzb[q]);
+        b0[q] = a0[q] * r8[q];
+      }
+      float wt = lane_above(wb[0]), bt = lane_above(b0[0]);
+      if (MZ && lane == 63) {
+        hte = h * (o.te + T0[V - 1]);
+        dze = fmaf(o.se - S0[V - 1], d.idz, dpie);
+        geb = o.ge;
+        web = fmaf(hte * ((o.pe - P0[V - 1]) * d.idz) + o.ge, dts, o.we);
+        wt = web;
+        bt = (0.5f * (wt * dze)) * r8e;
+      }
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        const bool lid = kl + q >= nz - 1;
+        const float w1 = lid ? 0.0f : (q < V - 1 ? wb[V - 1] : wt);
+        const float b1 = lid ? 0.0f : (q < V - 1 ? b0[V - 1] : bt);
+        htx1[q] = h * (o.t1[q] + T0[q]);
+        dsx1[q] = (o.s1[q] - S0[q]) * d.idx;
+        gu1[q] = o.gu[q];
+        ub1[q] = fmaf(fmaf(htx1[q], (o.p1[q] - P0[q]) * d.idx, o.gu[q]), dts, o.uf[q]);
+        const float du = ub1[q] * dsx1[q];
+        div0[q] = fmaf(w1 - wb[q], d.idz, fmaf(vb[1][q] - vb[0][q], d.idy, (ub1[q] - ul[q]) * d.idx));
+        const float z = quotient(fmaf(a0[q], r8[q], b1), rr[q], ir[q]);
+        const float advp = -(fmaf(0.5f, du + dl[q], 0.5f * (dv[1][q] + dv[0][q])) + z);
+        pa1[q] = pic[q] + S0[q];
+        const float dpdt = fmaf((float)(-kRd / kCv), pa1[q] * div0[q], advp);
+        pn[q] = fmaf(1.1f * dpdt, dts, P0[q]);
+        ul[q] = ub1[q];
+        dl[q] = du;
+        P0[q] = o.p1[q];
+        T0[q] = o.t1[q];
+        S0[q] = o.s1[q];
+      }
+    }
+    {
+      float* L = own + ((s + 1 - x0) & 1) * slab;
+#pragma unroll
+      for (int q = 0; q < V; ++q) L[q] = pn[q];
+    }
+    if (s < x1) {
+      if (s + 1 == 0 || s + 1 == nx) {
+        place(0);
+      } else {
+        pX += sxc;
+        tX += sxc;
+        sX += sxc;
+        uX += sxc;
+        vX += sxv;
+        wX += sxw;
+        guX += sxiu;
+        gvX += sxiv;
+        gwX += sxiw;
+      }
+      fetch(o);
+    }
+    // second substep: x face s, then pi' of cell s - 1
+    if (s >= x0) {
+      float pn2[V], us[V], un[V];
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        un[q] = fmaf(fmaf(htx[q], (pn[q] - pb[q]) * d.idx, gub[q]), dts, ub[q]);
+        const float du = un[q] * dsx[q];
+        const float div = fmaf(dwn[q], d.idz, fmaf(dvn[q], d.idy, (un[q] - ulb[q]) * d.idx));
+        const float advp = -(fmaf(0.5f, du + dlb[q], hdv[q]) + zz[q]);
+        const float dpdt = fmaf((float)(-kRd / kCv), pab[q] * div, advp);
+        pn2[q] = fmaf(1.1f * dpdt, dts, pb[q]);
+        us[q] = ulb[q];
+        ulb[q] = un[q];
+        dlb[q] = du;
+      }
+      if (second) {
+        const int x = s - 1;
+        if (x >= 4 && x < nx - 3 && j >= 4 && j < ny - 3) {
+          float* poX = a.po + (long)(x + 3) * sxc;
+          float* uoX = a.uo + (long)(x + 3) * sxc;
+          st_levels<V>(poX, oc, ls, pn2);
+          st_levels<V>(uoX, oc, ls, us);
+          if (ls.first || ls.last) {
+            st_ghosts<V>(poX, oc, ls, pn2);
+            st_ghosts<V>(uoX, oc, ls, us);
+          }
+        } else {
+          st_images<V, false>(a.po, sxc, syc, x, nx, false, j, ny, false, eK, ls, pn2);
+          st_images<V, false>(a.uo, sxc, syc, x, nx, true, j, ny, false, eK, ls, us);
+          if (x == nx - 1) st_images<V, false>(a.uo, sxc, syc, nx, nx, true, j, ny, false, eK, ls, un);
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      pb[q] = pn[q];
+      pab[q] = pa1[q];
+      ub[q] = ub1[q];
+      gub[q] = gu1[q];
+      htx[q] = htx1[q];
+      dsx[q] = dsx1[q];
+    }
+    __syncthreads();
+  }
+}
+
+// Columns of at most two waves; a taller one would leave a workgroup too few rows.
+inline bool acoustic2_ok(const Dims& d) { return d.nz <= 256; }
+
+// ROWS: two levels per lane need 142 to 160 VGPRs, three waves per SIMD, so one workgroup of
+// twelve waves fills a CU; with one level (87 VGPRs) two workgroups of eight.  The march is as
+// long as leaves every CU its workgroups once: a second, partly filled round costs more than
+// the two positions that a longer march saves.
+template <int V, bool MZ, int ROWS>
+inline void launch_acoustic2_v(const Dims& d, const AcousticArgs& a, hipStream_t st) {
+  constexpr int kLanes = MZ ? 128 : 64;
+  const int strips = (d.ny + ROWS - 3) / (ROWS - 2);
+  const int parts = std::max(1, std::min(d.nx, (V == 1 ? 512 : 256) / strips));
+  const int ax = (d.nx + parts - 1) / parts;
+  const dim3 g(strips, (d.nx + ax - 1) / ax), b(kLanes, ROWS);
+  const size_t lds = (size_t)2 * ROWS * kLanes * V * sizeof(float);
+  LEX_LAUNCH(KID_ACOUSTIC2, (k_acoustic2<V, MZ, kLanes * ROWS>), g, b, lds, st, d, a, ax);
+}
+inline void launch_acoustic2(const Dims& d, const AcousticArgs& a, hipStream_t st) {
+  if (d.nz <= 64)
+    launch_acoustic2_v<1, false, 8>(d, a, st);
+  else if (d.nz <= 128)
+    launch_acoustic2_v<2, false, 12>(d, a, st);
+  else
+    launch_acoustic2_v<2, true, 6>(d, a, st);
 }
 
 }  // namespace lex

@@ -485,7 +485,7 @@ int rk3_step(const Dims& d, const O& o, const B& b, float* const* state, char* w
     }
     float* in[4] = {X0[1], X0[2], X0[3], X0[4]};
     // the fused path advances two substeps per launch while two remain
-    const bool pairs = (o.solver != 3) && (o.impl == 0) && acoustic2_pays(d);
+    const bool pairs = (o.solver != 3) && (o.impl == 0) && acoustic2_ok(d);
     for (int t = 0; t < nsub;) {
       const int tn = t + ((pairs && t + 1 < nsub) ? 2 : 1);
       float* out[4];
@@ -506,9 +506,8 @@ int rk3_step(const Dims& d, const O& o, const B& b, float* const* state, char* w
         LEX_LAUNCH(KID_ACOUSTIC, k_acoustic_m, ag, dim3(64, 4, 1), 0, st, d, rc, b.pi0, in[0], in[1], in[2], in[3],
                    src[4], ru, rv, rw, tr, out[0], out[1], out[2], out[3], dts);
       } else if (tn == t + 2) {
-        LEX_LAUNCH(KID_ACOUSTIC2, k_acoustic2, acoustic2_grid(d), dim3(acoustic2_lanes(d), acoustic2_rows(d), 1),
-                   acoustic2_lds(d), st, d, rc, b.pi0, in[0], in[1], in[2], in[3], src[4], ru, rv, rw, tr, out[0],
-                   out[1], out[2], out[3], dts, acoustic2_ax(d));
+        launch_acoustic2(d, AcousticArgs{rc, b.pi0, in[0], in[1], in[2], in[3], src[4], ru, rv, rw, tr, out[0], out[1],
+                                         out[2], out[3], dts}, st);
       } else {
         launch_acoustic(d, AcousticArgs{rc, b.pi0, in[0], in[1], in[2], in[3], src[4], ru, rv, rw, tr, out[0], out[1],
                                         out[2], out[3], dts}, st);

@@ -70,6 +70,36 @@ def test_acoustic_substep_against_oracle(shape):
         check_fp32(from_dev(got), r64, r32, name)
 
 
+# one and two levels per lane, columns of one wave and of two, full and partial strips of
+# rows, marches of one and of several cells, the last one shorter
+@pytest.mark.parametrize("shape", [(6, 6, 24), (7, 13, 64), (100, 13, 40), (17, 9, 65), (33, 21, 128), (9, 7, 129),
+                                   (20, 9, 256), (181, 147, 71), (300, 60, 33)], ids=str)
+def test_acoustic_pair_is_two_substeps(shape):
+    """Two substeps in one launch equal two launches bit for bit; the input's ghosts are not
+    periodic images."""
+    import torch
+    from lex_amd import _lib
+    nx, ny, nz = shape
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    R = lambda s, *n: s * torch.randn(*n, generator=gen, device="cuda")  # noqa: E731
+    u, v = R(2.0, nx + 7, ny + 6, nz + 2), R(2.0, nx + 6, ny + 7, nz + 2)
+    w, p = R(2.0, nx + 6, ny + 6, nz + 3), R(1e-5, nx + 6, ny + 6, nz + 2)
+    tr, ps = 300.0 + R(1.0, nx + 6, ny + 6, nz + 2), p + R(1e-6, nx + 6, ny + 6, nz + 2)
+    ru, rv, rw = R(1e-2, nx + 1, ny, nz), R(1e-2, nx, ny + 1, nz), R(1e-2, nx, ny, nz + 1)
+    rho, pi0 = 1.0 + 0.1 * R(1.0, nz + 2).abs(), 0.9 + R(1e-2, nz + 2)
+    g = _lib.grid(nx, ny, nz, 100.0, 110.0, 90.0)
+
+    def call(name, state):
+        out = [torch.full_like(t, float("nan")) for t in state]
+        ins = (rho, pi0, *state, ps, ru, rv, rw, tr)
+        _lib.call(name, g, *[_lib.ptr(t) for t in ins], 0.1, *[_lib.ptr(t) for t in out], _lib.stream())
+        return out
+
+    want = call("lex_acoustic_substep", call("lex_acoustic_substep", (u, v, w, p)))
+    for name, a, b in zip("u v w p".split(), call("lex_acoustic_substep_pair", (u, v, w, p)), want):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num()), name
+
+
 # one block, several with a last one partly filled, exactly two cells per thread, and the
 # loop past the two cells a thread requests ahead (more than 1024 blocks of 512 cells)
 @pytest.mark.parametrize("shape", [(6, 6, 6), (19, 23, 17), (32, 32, 64), (96, 96, 60)], ids=str)
