@@ -488,13 +488,6 @@ __global__ void k_set_w_bc(Dims d, float* __restrict__ w) {
   w[b + d.nz + 2] = 0.0f;
 }
 
-// ----------------------------------------------------------------------------------
-// S1 arithmetic of one cell (one_step_integration.py:528-553): the six face velocities
-// after pressure_gradient_force + rhs, set_w_bc at the surface and lid, the divergence,
-// advection_pi with the fixed pi* and the damped pi' update.  Operands: the cell's faces
-// (u0/u1 lower/upper x face, ...), the rhs on those faces, the 7-point stencils of pi',
-// theta_rho and pi*, and the rho0 / pi0 column values at levels K-1, K, K+1.
-// ----------------------------------------------------------------------------------
 // x / r from the correctly rounded reciprocal ir of r: the product and one residual
 // correction, which is the correctly rounded quotient where nothing under- or overflows
 // (three operations instead of the ten of an IEEE division; r is a density).

@@ -9,6 +9,7 @@
 //                   (kmv, khv) for tau13, tau23 and the z scalar fluxes.  turb_opt 1 passes
 //                   the same array for both.
 #pragma once
+#include <algorithm>
 #include "lex_common.hpp"
 
 namespace lex {
@@ -463,10 +464,19 @@ inline size_t smag_fused_lds(const Dims& d, bool aniso) {
   const int nzl = 64 * ((d.nz + 63) / 64);
   return sizeof(float) * (size_t)smag_fused_rows(d) * nzl * (aniso ? 23 : 20);
 }
-constexpr int kSmagAx = 16;   // x cells per workgroup
+// Cells along x per workgroup: the fewest with which all workgroups are resident at once (24
+// waves per CU), at most 16 (two of ax + 2 planes are recomputed).  us of a step with 2, 4, 8
+// and 16 cells: 40x40x40 143, 150, 163, 192; 96x96x48 289, 287, 297, 327; 128x128x64 403, 388,
+// 398, 420; 192x160x96 1211, 1198, 1186, 1180.
+inline int smag_fused_ax(const Dims& d) {
+  const int ty = smag_fused_rows(d) - 2, strips = (d.ny + ty - 1) / ty;
+  const int threads = 64 * ((d.nz + 63) / 64) * smag_fused_rows(d);
+  const int parts = std::max(1, 256 * (1536 / threads) / strips);
+  return std::min(16, (d.nx + parts - 1) / parts);
+}
 inline dim3 smag_fused_grid(const Dims& d) {
-  const int ty = smag_fused_rows(d) - 2;
-  return dim3((d.ny + ty - 1) / ty, (d.nx + kSmagAx - 1) / kSmagAx, 1);
+  const int ty = smag_fused_rows(d) - 2, ax = smag_fused_ax(d);
+  return dim3((d.ny + ty - 1) / ty, (d.nx + ax - 1) / ax, 1);
 }
 
 template <bool ANISO>
@@ -475,7 +485,7 @@ __global__ void __launch_bounds__(768, 6) k_smag_fused(Dims d, const float* __re
                                                       const float* __restrict__ th, const float* __restrict__ qv,
                                                       float csgs2, float prandtl, float csq, SgsScalars S,
                                                       float* __restrict__ su, float* __restrict__ sv,
-                                                      float* __restrict__ sw) {
+                                                      float* __restrict__ sw, int ax) {
 #pragma clang fp contract(off)
   extern __shared__ float lds[];
   const int nzl = blockDim.x, TYT = blockDim.y;
@@ -493,7 +503,7 @@ __global__ void __launch_bounds__(768, 6) k_smag_fused(Dims d, const float* __re
   const int lane = threadIdx.x, row = threadIdx.y;
   const TileId tb = xcd_tile();
   const int j0 = tb.x * (TYT - 2);
-  const int x0 = tb.y * kSmagAx, x1 = min(x0 + kSmagAx, d.nx);
+  const int x0 = tb.y * ax, x1 = min(x0 + ax, d.nx);
   const int nz = d.nz;
   const int j = j0 - 1 + row;                 // -1 .. j0+TYT-2 (rows past ny are never read)
   // halo rows and planes are evaluated at their periodic images (the interior cell's own

@@ -375,10 +375,12 @@ int rk3_step(const Dims& d, const O& o, const B& b, float* const* state, char* w
         const dim3 fbk(64 * ((d.nz + 63) / 64), smag_fused_rows(d), 1);
         if (an)
           LEX_LAUNCH(KID_SMAG_ONE, k_smag_fused<true>, smag_fused_grid(d), fbk, smag_fused_lds(d, true), st, d, rc,
-                     src[1], src[2], src[3], src[0], src[5], cg * cg, o.prandtl, o.cs * o.cs, SS, su, sv, sw);
+                     src[1], src[2], src[3], src[0], src[5], cg * cg, o.prandtl, o.cs * o.cs, SS, su, sv, sw,
+                     smag_fused_ax(d));
         else
           LEX_LAUNCH(KID_SMAG_ONE, k_smag_fused<false>, smag_fused_grid(d), fbk, smag_fused_lds(d, false), st, d, rc,
-                     src[1], src[2], src[3], src[0], src[5], cg * cg, o.prandtl, o.cs * o.cs, SS, su, sv, sw);
+                     src[1], src[2], src[3], src[0], src[5], cg * cg, o.prandtl, o.cs * o.cs, SS, su, sv, sw,
+                     smag_fused_ax(d));
       } else if (o.impl != 1) {
         // the fused paths when the one-pass kernel does not apply (nz mod 64 of 1 or 2):
         // deformation, N^2 and the coefficients in one pass writing the stresses and

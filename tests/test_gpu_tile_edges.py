@@ -100,6 +100,13 @@ def test_acoustic_pair_is_two_substeps(shape):
         assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num()), name
 
 
+# marches of 2, 4 and 5 cells, the last one shorter
+@pytest.mark.parametrize("shape", [(101, 90, 24), (110, 130, 64), (97, 91, 70)], ids=str)
+def test_smagorinsky_marches_equal_routine_chain(shape):
+    from tests.test_gpu_step import test_fused_smagorinsky_equals_routine_chain as chain
+    chain(shape, 1)
+
+
 # one block, several with a last one partly filled, exactly two cells per thread, and the
 # loop past the two cells a thread requests ahead (more than 1024 blocks of 512 cells)
 @pytest.mark.parametrize("shape", [(6, 6, 6), (19, 23, 17), (32, 32, 64), (96, 96, 60)], ids=str)
