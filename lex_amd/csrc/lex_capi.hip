@@ -430,8 +430,7 @@ int lex_acoustic_substep_implicit(const lex_grid_t* g, const float* r, const flo
     return fail(-1, "lex_acoustic_substep_implicit: outputs must not alias inputs%s");
   if (g->nz < 2 || g->nz > 256) return fail(-1, "lex_acoustic_substep_implicit: nz must be 2..256%s");
   Dims d = mkdims(g);
-  hipLaunchKernelGGL(k_acoustic_vi, dim3(d.ny, d.nx, 1), dim3(acoustic_vi_lanes(d)), acoustic_vi_lds(d), S(stream),
-                     d, r, pi0, u, v, w, p, ps, ru, rv, rw, tr, uo, vo, wo, po, dts, alpha);
+  launch_acoustic_vi(d, AcousticArgs{r, pi0, u, v, w, p, ps, ru, rv, rw, tr, uo, vo, wo, po, dts}, alpha, S(stream));
   return check_launch("lex_acoustic_substep_implicit");
 }
 

@@ -107,6 +107,39 @@ def test_smagorinsky_marches_equal_routine_chain(shape):
     chain(shape, 1)
 
 
+# one and two levels per lane, the smallest and the fullest columns of each, one level left
+# over, marches of one and of several cells
+@pytest.mark.parametrize("shape", [(8, 9, 6), (17, 9, 64), (9, 7, 65), (9, 8, 127), (12, 11, 128), (161, 160, 33)],
+                         ids=str)
+def test_implicit_substep_against_oracle(shape):
+    """One vertically implicit substep against the FP64 oracle (a Thomas solve there); error
+    within 8x the FP32 oracle's own, as for the other operators."""
+    import torch
+    from lex_amd import _lib
+    from oracle import lex_oracle as o
+    from tests._helpers import check_fp32
+    nx, ny, nz = shape
+    gr, phys, base = random_state(nx, ny, nz, seed=5, vel=2.0)
+    rng = np.random.default_rng(7)
+    th, u, v, w, p = (np.asarray(a, np.float32) for a in phys[:5])
+    ps = np.asarray(p + rng.normal(0, 1e-6, p.shape), np.float32)
+    ru, rv, rw = (np.asarray(rng.normal(0, 1e-2, s), np.float32)
+                  for s in ((nx + 1, ny, nz), (nx, ny + 1, nz), (nx, ny, nz + 1)))
+    rho, pi0 = (np.asarray(base[q], np.float32) for q in (1, 3))
+    ref = []
+    for dt in (np.float64, np.float32):
+        f = lambda a: np.asarray(a, dt)  # noqa: E731
+        ref.append(o.sound_implicit_rk_step(f(u), f(v), f(w), f(pi0), f(p), f(ps), f(ru), f(rv), f(rw), f(th), f(rho),
+                                            1, 0.2, gr))
+    ins = [to_dev(a) for a in (rho[3, 3], pi0[3, 3], u, v, w, p, ps, ru, rv, rw, th)]
+    out = [torch.full_like(t, float("nan")) for t in ins[2:6]]
+    g = _lib.grid(nx, ny, nz, gr.dx, gr.dy, gr.dz)
+    _lib.call("lex_acoustic_substep_implicit", g, *[_lib.ptr(t) for t in ins], 0.2, 0.6, *[_lib.ptr(t) for t in out],
+              _lib.stream())
+    for name, got, a0, r64, r32 in zip("u v w p".split(), out, (u, v, w, p), *ref):
+        check_fp32(from_dev(got) - a0, r64 - a0, r32 - a0, name)
+
+
 # one block, several with a last one partly filled, exactly two cells per thread, and the
 # loop past the two cells a thread requests ahead (more than 1024 blocks of 512 cells)
 @pytest.mark.parametrize("shape", [(6, 6, 6), (19, 23, 17), (32, 32, 64), (96, 96, 60)], ids=str)
