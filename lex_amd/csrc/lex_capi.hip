@@ -1106,7 +1106,7 @@ void launch_fwd(int nx, int ny, int nz, const void* x, const void* wp, const flo
                        bias, mode, cout_real, (__bf16*)y, yf, pre);
   }
 }
-// workgroups of k_conv3_wgrad: one per CU (the accumulators fill the register file)
+// workgroups of k_conv3_wgrad: one of eight waves per CU (each adds a slot of partial sums)
 inline unsigned wgrad_blocks(int nx, int ny, int nz) {
   long nt = (long)((nx + CTX - 1) / CTX) * ((ny + CTY - 1) / CTY) * ((nz + CTZ - 1) / CTZ);
   return (unsigned)(nt < 256 ? nt : 256);
@@ -1117,7 +1117,7 @@ template <int CI, int CO>
 void launch_wgrad(int nx, int ny, int nz, const void* x, const void* g, float* dw, float* part, float* db,
                   int cout, hipStream_t st) {
   const unsigned nb = wgrad_blocks(nx, ny, nz);
-  hipLaunchKernelGGL((k_conv3_wgrad<CI, CO>), dim3(nb), dim3(256), 0, st, nx, ny, nz, (const __bf16*)x,
+  hipLaunchKernelGGL((k_conv3_wgrad<CI, CO>), dim3(nb), dim3(512), 0, st, nx, ny, nz, (const __bf16*)x,
                      (const __bf16*)g, part, db ? 1 : 0);
   const int n = 27 * CI * CO, n2 = db ? cout : 0;
   hipLaunchKernelGGL(k_partial_sum, dim3((n + n2 + 63) / 64), dim3(64), 0, st, (int)nb, n, n + CO,

@@ -523,7 +523,7 @@ inline int conv_rows_resident() {
 // Weight gradient: dW[tap][c][n] += sum_p X[p + o(tap)][c] * G[p][n] over the cells of
 // the grid (G: BF16 gradient of the pre-activation, COUT channels).  Workgroups loop
 // over output tiles and store their FP32 partial sums (all 27 CIN COUT of them) in the
-// slot of part that belongs to the workgroup; k_wgrad_reduce then adds the slots in
+// slot of part that belongs to the workgroup; k_partial_sum then adds the slots in
 // workgroup order, so the result does not depend on the order the workgroups ran in.
 //
 // The reduction runs over cells, so an MFMA operand lane needs 8 consecutive cells of
@@ -535,146 +535,203 @@ inline int conv_rows_resident() {
 // offset 0, where it is stored).
 constexpr int XR = 24;
 
-__device__ __forceinline__ bf16x8 xrun_window(const __bf16* __restrict__ row, int hz, int dz) {
+// Eight waves; tile t + 1 is on its way to registers while tile t is multiplied.  The cells of
+// a tile are halved between waves 0-3 and 4-7; within a half a wave takes some of the nine
+// (dx, dy) pairs and, with 32 input channels, one of the two 16-channel groups: the three dz of
+// a pair come from the same aligned read and its two neighbouring dwords, and the G operands
+// serve all of a wave's taps.  The two waves of a SIMD hold the larger and the smaller share of
+// pairs.  Neighbouring cells are transposed two at a time, so that LDS takes 4-byte writes.
+// Four waves, one per SIMD (487 VGPRs), that took single taps waited for the tile's loads, read
+// G again for every tap and wrote 2-byte scatters: us per call (22 to 25 of them around the
+// kernel) at 96x96x48, 16->16, 16->32, 32->16 and 32->32 channels, 67, 74, 110 and 127; now 35,
+// 42, 46 and 56.
+// Workgroup b stores its partial sums at part + b * (27 CIN COUT + COUT): the weights' (the two
+// halves added through LDS), then (with_bias) the bias gradient's, which rides along: once a G
+// tile is in LDS, the 512 / COUT threads of each channel row add their consecutive cells of it,
+// in order, to one running FP32 sum each; at the end the sums of a channel are added in thread
+// order.
+// element j of lo and of hi in one word
+__device__ __forceinline__ unsigned pair16(const bf16x8& lo, const bf16x8& hi, int j) {
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-  const u32x4 c = *(const u32x4*)(row + 8 + hz);
-  if (dz == 0) return __builtin_bit_cast(bf16x8, c);
-  u32x4 r;
-  if (dz < 0) {
-    const unsigned lo = *(const unsigned*)(row + 6 + hz);  // elements 6+hz, 7+hz
-    r[0] = __builtin_amdgcn_alignbyte(c[0], lo, 2);
-    r[1] = __builtin_amdgcn_alignbyte(c[1], c[0], 2);
-    r[2] = __builtin_amdgcn_alignbyte(c[2], c[1], 2);
-    r[3] = __builtin_amdgcn_alignbyte(c[3], c[2], 2);
-  } else {
-    const unsigned hi = *(const unsigned*)(row + (16 + hz) % XR);  // element 16+hz (or the upper halo)
-    r[0] = __builtin_amdgcn_alignbyte(c[1], c[0], 2);
-    r[1] = __builtin_amdgcn_alignbyte(c[2], c[1], 2);
-    r[2] = __builtin_amdgcn_alignbyte(c[3], c[2], 2);
-    r[3] = __builtin_amdgcn_alignbyte(hi, c[3], 2);
-  }
-  return __builtin_bit_cast(bf16x8, r);
+  const u32x4 a = __builtin_bit_cast(u32x4, lo), b = __builtin_bit_cast(u32x4, hi);
+  return __builtin_amdgcn_perm(b[j >> 1], a[j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
 }
 
-// Workgroup b stores its partial sums at part + b * (27 CIN COUT + COUT): the weights', then
-// (with_bias) the bias gradient's, which rides along: once a G tile is in LDS, the 256 /
-// COUT threads of each channel row add COUT consecutive cells of it, in order, to one
-// running FP32 sum each; at the end the sums of a channel are added in thread order.
 template <int CIN, int COUT>
-__global__ __launch_bounds__(256) void k_conv3_wgrad(int nx, int ny, int nz, const __bf16* __restrict__ X,
+__global__ __launch_bounds__(512) void k_conv3_wgrad(int nx, int ny, int nz, const __bf16* __restrict__ X,
                                                      const __bf16* __restrict__ G, float* __restrict__ part,
                                                      int with_bias) {
   static_assert(CTZ == 16 && XR == 24, "z-run layout assumes a 16-cell z tile");
-  constexpr int MT = COUT / 16, NT = CIN / 16, TPW = 7;  // taps per wave: 7, 7, 7, 6
-  constexpr int NCELL = CTX * CTY * CTZ;
-  constexpr int TPC = 256 / COUT;   // bias: threads per channel row, COUT cells each
-  static_assert(NCELL == 256 && NCELL % TPC == 0, "bias sums: one 256-cell tile per 256 threads");
-  float bsum = 0.f;
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  constexpr int NCELL = CTX * CTY * CTZ, NL = HX * HY, NTH = 512;
+  constexpr int MT = COUT / 16, NT = CIN / 16, NG = 4 / NT, PP = (9 + NG - 1) / NG;
+  constexpr int TPC = NTH / COUT;   // bias: threads per channel row
+  static_assert(NCELL == 256 && NCELL % (8 * TPC) == 0, "bias sums: whole 16-byte reads of a 256-cell row");
   // channel rows padded to an odd multiple of 16 bytes (modulo 256): the 16 lanes of an
   // operand read take 16 different channel rows at one offset, which then fall on 16
   // distinct bank groups instead of 1 (G rows of 512 bytes) or 4 (X rows of 1728)
-  constexpr int XS = HX * HY * XR + 8, GS = NCELL + 8;   // row strides in elements
+  constexpr int XS = NL * XR + 8, GS = NCELL + 8;   // row strides in elements
   static_assert((XS * 2) % 32 == 16 && (GS * 2) % 32 == 16, "odd multiples of 16 bytes");
   __shared__ __attribute__((aligned(16))) __bf16 xt[CIN * XS];  // [c][hx][hy][z-run]
   __shared__ __attribute__((aligned(16))) __bf16 gt[COUT * GS];  // [n][cell]
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, m = l & 15, g = l >> 4;
-  f32x4 acc[TPW][MT][NT];
+  static_assert(4 * 64 * 3 * MT * 4 * sizeof(float) <= sizeof(xt), "the halves are added through the X tile");
+  const int tid = threadIdx.x, l = tid & 63, m = l & 15, g = l >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), half = w >> 2, ct = NT == 2 ? w & 1 : 0;
+  const int pg0 = NT == 2 ? (w >> 1) & 1 : w & 3, pg = half ? NG - 1 - pg0 : pg0;
+  f32x4 acc[PP][3][MT];
 #pragma unroll
-  for (int a = 0; a < TPW; ++a)
-    for (int b = 0; b < MT; ++b)
-      for (int c = 0; c < NT; ++c) acc[a][b][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < PP; ++i)
+    for (int z = 0; z < 3; ++z)
+      for (int mt = 0; mt < MT; ++mt) acc[i][z][mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float bsum = 0.f;
+
+  // items of a tile: pairs of cells along z, and the two z ends of every halo line
+  constexpr int XP = NL * (CTZ / 2) * (CIN / 8), XE = NL * 2 * (CIN / 8), GP = NCELL / 2 * (COUT / 8);
+  constexpr int NXP = (XP + NTH - 1) / NTH, NXE = (XE + NTH - 1) / NTH, NGP = (GP + NTH - 1) / NTH;
+  bf16x8 xp[NXP][2], xe[NXE], gp[NGP][2];
   const int tz = (nz + CTZ - 1) / CTZ, ty = (ny + CTY - 1) / CTY, tx = (nx + CTX - 1) / CTX;
   const int ntiles = tx * ty * tz;
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+  auto ld = [&](const __bf16* f, int ch, int x, int y, int z, int c0) {
+    bf16x8 v = {};
+    if (x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz)
+      v = *(const bf16x8*)(f + (((long)x * ny + y) * nz + z) * ch + c0);
+    return v;
+  };
+  auto fetch = [&](int tile) {
     const int z0 = (tile % tz) * CTZ, y0 = ((tile / tz) % ty) * CTY, x0 = (tile / (tz * ty)) * CTX;
-    __syncthreads();
-    // X halo tile: one 16-byte load = 8 channels of one cell, scattered to 8 channel rows
-    // (neighbouring lanes take neighbouring cells, so their 2-byte stores share banks
-    // only pairwise)
-    for (int e = threadIdx.x; e < HX * HY * HZ * (CIN / 8); e += 256) {
-      const int cell = e % (HX * HY * HZ), cg = e / (HX * HY * HZ);
-      const int hz = cell % HZ, hy = (cell / HZ) % HY, hx = cell / (HZ * HY);
-      const int gx = x0 + hx - 1, gy = y0 + hy - 1, gz = z0 + hz - 1;
-      bf16x8 v;
-      if (gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz) {
-        v = *(const bf16x8*)(X + (((long)gx * ny + gy) * nz + gz) * CIN + 8 * cg);
-      } else {
-        for (int j = 0; j < 8; ++j) v[j] = (__bf16)0.0f;
-      }
-      __bf16* dst = xt + (8 * cg) * XS + (hx * HY + hy) * XR + (hz == HZ - 1 ? 0 : 7 + hz);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) dst[j * XS] = v[j];
+    for (int q = 0; q < NXP; ++q) {
+      const int e = tid + q * NTH;
+      if (e >= XP) break;
+      const int zp = e % (CTZ / 2), line = (e / (CTZ / 2)) % NL, cg = e / (CTZ / 2 * NL);
+      const int x = x0 + line / HY - 1, y = y0 + line % HY - 1, z = z0 + 2 * zp;
+      xp[q][0] = ld(X, CIN, x, y, z, 8 * cg);
+      xp[q][1] = ld(X, CIN, x, y, z + 1, 8 * cg);
     }
-    // G tile: 8 channels of one cell per load, scattered to 8 channel rows
-    for (int e = threadIdx.x; e < NCELL * (COUT / 8); e += 256) {
-      const int cell = e % NCELL, ng = e / NCELL;
-      const int hz = cell % CTZ, hy = (cell / CTZ) % CTY, hx = cell / (CTZ * CTY);
-      const int gx = x0 + hx, gy = y0 + hy, gz = z0 + hz;
-      bf16x8 v;
-      if (gx < nx && gy < ny && gz < nz) {
-        v = *(const bf16x8*)(G + (((long)gx * ny + gy) * nz + gz) * COUT + 8 * ng);
-      } else {
-        for (int j = 0; j < 8; ++j) v[j] = (__bf16)0.0f;
-      }
 #pragma unroll
-      for (int j = 0; j < 8; ++j) gt[(8 * ng + j) * GS + cell] = v[j];
+    for (int q = 0; q < NXE; ++q) {
+      const int e = tid + q * NTH;
+      if (e >= XE) break;
+      const int hi = e & 1, line = (e >> 1) % NL, cg = (e >> 1) / NL;
+      xe[q] = ld(X, CIN, x0 + line / HY - 1, y0 + line % HY - 1, hi ? z0 + CTZ : z0 - 1, 8 * cg);
     }
+#pragma unroll
+    for (int q = 0; q < NGP; ++q) {
+      const int e = tid + q * NTH;
+      if (e >= GP) break;
+      const int cell = 2 * (e % (NCELL / 2)), ng = e / (NCELL / 2);
+      const int x = x0 + cell / (CTY * CTZ), y = y0 + (cell / CTZ) % CTY, z = z0 + cell % CTZ;
+      gp[q][0] = ld(G, COUT, x, y, z, 8 * ng);
+      gp[q][1] = ld(G, COUT, x, y, z + 1, 8 * ng);
+    }
+  };
+  auto place = [&]() {
+#pragma unroll
+    for (int q = 0; q < NXP; ++q) {
+      const int e = tid + q * NTH;
+      if (e >= XP) break;
+      const int zp = e % (CTZ / 2), line = (e / (CTZ / 2)) % NL, cg = e / (CTZ / 2 * NL);
+      __bf16* dst = xt + (8 * cg) * XS + line * XR + 8 + 2 * zp;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) *(unsigned*)(dst + j * XS) = pair16(xp[q][0], xp[q][1], j);
+    }
+#pragma unroll
+    for (int q = 0; q < NXE; ++q) {
+      const int e = tid + q * NTH;
+      if (e >= XE) break;
+      const int hi = e & 1, line = (e >> 1) % NL, cg = (e >> 1) / NL;
+      __bf16* dst = xt + (8 * cg) * XS + line * XR + (hi ? 0 : 7);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) dst[j * XS] = xe[q][j];
+    }
+#pragma unroll
+    for (int q = 0; q < NGP; ++q) {
+      const int e = tid + q * NTH;
+      if (e >= GP) break;
+      const int cell = 2 * (e % (NCELL / 2)), ng = e / (NCELL / 2);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) *(unsigned*)(gt + (8 * ng + j) * GS + cell) = pair16(gp[q][0], gp[q][1], j);
+    }
+  };
+  const int step = gridDim.x;
+  fetch(blockIdx.x);
+  for (int tile = blockIdx.x; tile < ntiles; tile += step) {
+    place();
     __syncthreads();
+    if (tile + step < ntiles) fetch(tile + step);
     if (with_bias) {   // uniform
-      const __bf16* row = gt + (threadIdx.x / TPC) * GS + (threadIdx.x % TPC) * COUT;
+      const __bf16* row = gt + (tid / TPC) * GS + (tid % TPC) * (NCELL / TPC);
 #pragma unroll
-      for (int r = 0; r < COUT / 8; ++r) {
+      for (int r = 0; r < NCELL / TPC / 8; ++r) {
         const bf16x8 v = *(const bf16x8*)(row + 8 * r);
 #pragma unroll
         for (int j = 0; j < 8; ++j) bsum += (float)v[j];
       }
     }
+#pragma unroll 1
+    for (int ks = 4 * half; ks < 4 * half + 4; ++ks) {
+      const int k0 = ks * 32 + 8 * g;  // 8 consecutive cells along z of one (hx, hy) line
+      const int hx = ks >> 1, hy = 2 * (ks & 1) + (g >> 1), hz = 8 * (g & 1);
+      bf16x8 a[MT];
 #pragma unroll
-    for (int q = 0; q < TPW; ++q) {
-      const int tap = w + 4 * q;
-      if (tap > 26) continue;
-      const int dx = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dz = tap % 3 - 1;
-      for (int ks = 0; ks < NCELL / 32; ++ks) {
-        const int k0 = ks * 32 + 8 * g;  // 8 consecutive cells along z of one (hx, hy) line
-        const int hx = k0 / (CTY * CTZ), hy = (k0 / CTZ) % CTY, hz = k0 % CTZ;
-        bf16x8 a[MT], b[NT];
+      for (int mt = 0; mt < MT; ++mt) a[mt] = *(const bf16x8*)(gt + (mt * 16 + m) * GS + k0);
+      const __bf16* xc = xt + (ct * 16 + m) * XS + (hx * HY + hy) * XR;
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) a[mt] = *(const bf16x8*)(gt + (mt * 16 + m) * GS + k0);
-        const int rb = (hx + 1 + dx) * HY + (hy + 1 + dy);
+      for (int i = 0; i < PP; ++i) {
+        const int p = pg + i * NG;
+        if (p >= 9) break;   // uniform over the wave
+        const __bf16* row = xc + ((p / 3) * HY + p % 3) * XR;
+        const u32x4 c = *(const u32x4*)(row + 8 + hz);
+        const unsigned lo = *(const unsigned*)(row + 6 + hz);         // elements 6 + hz, 7 + hz
+        const unsigned hi = *(const unsigned*)(row + (hz ? 0 : 16));  // element 16 + hz, or the upper halo
+        u32x4 wl, wh;
+        wl[0] = __builtin_amdgcn_alignbyte(c[0], lo, 2);
+        wh[3] = __builtin_amdgcn_alignbyte(hi, c[3], 2);
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) b[nt] = xrun_window(xt + (nt * 16 + m) * XS + rb * XR, hz, dz);
+        for (int j = 0; j < 3; ++j) wl[j + 1] = wh[j] = __builtin_amdgcn_alignbyte(c[j + 1], c[j], 2);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt) acc[q][mt][nt] = mfma16(a[mt], b[nt], acc[q][mt][nt]);
+        for (int mt = 0; mt < MT; ++mt) {
+          acc[i][0][mt] = mfma16(a[mt], __builtin_bit_cast(bf16x8, wl), acc[i][0][mt]);
+          acc[i][1][mt] = mfma16(a[mt], __builtin_bit_cast(bf16x8, c), acc[i][1][mt]);
+          acc[i][2][mt] = mfma16(a[mt], __builtin_bit_cast(bf16x8, wh), acc[i][2][mt]);
+        }
       }
     }
+    __syncthreads();
   }
   float* dW = part + (long)blockIdx.x * (27 * CIN * COUT + COUT);
+  float* red = reinterpret_cast<float*>(xt);   // the X tile is no longer read
   if (with_bias) {
-    float* red = reinterpret_cast<float*>(xt);   // the X tile is no longer read
+    red[tid] = bsum;
     __syncthreads();
-    red[threadIdx.x] = bsum;
-    __syncthreads();
-    if (threadIdx.x < COUT) {
+    if (tid < COUT) {
       float s = 0.f;
-      for (int i = 0; i < TPC; ++i) s += red[threadIdx.x * TPC + i];
-      dW[27 * CIN * COUT + threadIdx.x] = s;
+      for (int i = 0; i < TPC; ++i) s += red[tid * TPC + i];
+      dW[27 * CIN * COUT + tid] = s;
     }
+    __syncthreads();
   }
-  // D[row = n][col = c]: lane holds rows 4g+i of the M-tile, column m of the N-tile; the
-  // four waves' taps (w, w+4, ..) cover all 27, so every element of the slot is stored
+  // D[row = n][col = c]: lane holds rows 4g+i of the M-tile, column m of the N-tile
+  f32x4* share = reinterpret_cast<f32x4*>(red) + ((pg * NT + ct) * 3 * MT) * 64 + l;
 #pragma unroll
-  for (int q = 0; q < TPW; ++q) {
-    const int tap = w + 4 * q;
-    if (tap > 26) continue;
+  for (int i = 0; i < PP; ++i) {
+    const int p = pg + i * NG;
+    if (half) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-      for (int nt = 0; nt < NT; ++nt)
-        for (int i = 0; i < 4; ++i) {
-          const int n = mt * 16 + 4 * g + i, c = nt * 16 + m;
-          dW[((long)tap * CIN + c) * COUT + n] = acc[q][mt][nt][i];
+      for (int z = 0; z < 3; ++z)
+        for (int mt = 0; mt < MT; ++mt) share[(z * MT + mt) * 64] = acc[i][z][mt];
+    }
+    __syncthreads();
+    if (!half && p < 9) {
+#pragma unroll
+      for (int z = 0; z < 3; ++z)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          const f32x4 s = acc[i][z][mt] + share[(z * MT + mt) * 64];
+          *(f32x4*)(dW + ((long)(3 * p + z) * CIN + ct * 16 + m) * COUT + mt * 16 + 4 * g) = s;
         }
+    }
+    __syncthreads();
   }
 }
 

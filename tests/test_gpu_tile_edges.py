@@ -198,3 +198,27 @@ def test_convolution_march(shape, cin, cout, circular):
     yb, pre = sn.conv3d_fwd(xd, shape, W.cuda(), b.cuda(), gelu=False, out_fp32=False, want_pre=True, circular=circular)
     rel = lambda a: float((a.cpu().double().view(*shape, -1)[..., :cout] - ref).norm() / ref.norm())  # noqa: E731
     assert rel(yf) < 1e-5 and rel(pre) < 1e-5 and rel(yb) < 2.0 ** -8
+
+
+# less than a tile, one tile over and under in each direction, several tiles per workgroup
+@pytest.mark.parametrize("cin,cout", [(16, 16), (9, 32), (32, 11), (32, 32)])
+@pytest.mark.parametrize("shape", [(5, 6, 7), (9, 4, 16), (4, 9, 33), (50, 47, 18)], ids=str)
+def test_conv_weight_gradient(shape, cin, cout):
+    """Weight and bias gradient against FP64 sums of the same BF16 operands: FP32 sums of n
+    products, whose rounding grows like sqrt(n) of an ulp."""
+    import torch
+    from lex_amd import sgs_net as sn
+    nx, ny, nz = shape
+    n, cip, cop = nx * ny * nz, 16 * ((cin + 15) // 16), 16 * ((cout + 15) // 16)
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.randn(n, cip, device="cuda", generator=gen).to(torch.bfloat16)
+    gp = torch.randn(n, cop, device="cuda", generator=gen).to(torch.bfloat16)
+    dw, db = sn.conv3d_bwd_weight(x, gp, shape, cin, cout)
+    xp = torch.zeros(nx + 2, ny + 2, nz + 2, cin, dtype=torch.float64, device="cuda")
+    xp[1:-1, 1:-1, 1:-1] = x[:, :cin].double().view(nx, ny, nz, cin)
+    g64 = gp[:, :cout].double()
+    ref = torch.stack([xp[a:a + nx, b:b + ny, c:c + nz].reshape(n, cin).t() @ g64
+                       for a in range(3) for b in range(3) for c in range(3)])
+    tol = n ** 0.5 * 2.0 ** -24
+    assert float((dw.double() - ref).norm() / ref.norm()) <= tol
+    assert float((db.double() - g64.sum(0)).norm() / g64.sum(0).norm()) <= 4 * tol   # sums that cancel
