@@ -814,7 +814,7 @@ int lex_acoustic_substep_vjp(const lex_grid_t* g, const float* r, const float* p
                      (const float*)lpo, (const float*)luo, (const float*)lvo, (const float*)lwo, dts, 1, lu, lv, lw, lru,
                      lrv, lrw, lU, lV, lW);
   hipLaunchKernelGGL(k_acoustic_vjp_cells3, grd(d.nz, d.ny + 2, d.nx + 2), blk(), 0, st, d, r, u, v, w, p, ru, rv, rw,
-                     tr, (const float*)lpo, (const float*)lU, (const float*)lV, (const float*)lW, dts, lp, ltr, lps);
+                     tr, (const float*)lpo, (const float*)lU, (const float*)lV, (const float*)lW, dts, 1, lp, ltr, lps);
   return check_launch("lex_acoustic_substep_vjp");
 }
 
