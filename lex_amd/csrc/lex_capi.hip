@@ -1135,6 +1135,15 @@ static int conv_fwd(const char* name, int nx, int ny, int nz, int cin, int cout,
   // the GELU-gradient epilogue (mode 8) exists for 32 output channels in the marching kernel only
   if ((mode & 8) && (mode != 8 || cip > 32 || cop != 32 || !pre))
     return fail(-1, "%s: the fused GELU gradient needs <= 32 input and 17..32 output channels", name);
+  // the march copies 16-byte chunks of x into LDS: a view that starts elsewhere is moved first
+  SlotScratch sc;
+  if (((uintptr_t)x & 15) != 0 && cip <= 32 && cop <= 32) {
+    const size_t bytes = (size_t)nx * ny * nz * cip * 2;
+    if (sc.take(bytes, st) != hipSuccess) return fail(-4, "%s: no device memory for an aligned copy of x", name);
+    if (hipMemcpyAsync(sc.p, x, bytes, hipMemcpyDeviceToDevice, st) != hipSuccess)
+      return fail(-3, "%s: copying x failed", name);
+    x = sc.p;
+  }
 #define LEX_FWD(CI, CO) \
   if (cip == CI && cop == CO) { launch_fwd<CI, CO>(nx, ny, nz, x, wp, bias, mode, cout, y, yf, pre, st); return check_launch(name); }
   LEX_FWD(16, 16) LEX_FWD(16, 32) LEX_FWD(16, 64)

@@ -222,3 +222,23 @@ def test_conv_weight_gradient(shape, cin, cout):
     tol = n ** 0.5 * 2.0 ** -24
     assert float((dw.double() - ref).norm() / ref.norm()) <= tol
     assert float((db.double() - g64.sum(0)).norm() / g64.sum(0).norm()) <= 4 * tol   # sums that cancel
+
+
+def test_conv_of_an_unaligned_view():
+    """An input that starts two bytes off a 16-byte boundary gives the aligned input's bits."""
+    import torch
+    from lex_amd import _lib
+    nx, ny, nz, c = 9, 7, 18, 32
+    n = nx * ny * nz
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn(n * c, device="cuda", generator=gen).to(torch.bfloat16)
+    off = torch.empty(n * c + 1, dtype=torch.bfloat16, device="cuda")[1:].copy_(x)
+    assert off.data_ptr() % 16 == 2
+    w, b = torch.randn(27, c, c, device="cuda", generator=gen), torch.zeros(c, device="cuda")
+    wp = torch.empty(c * 27 * c, dtype=torch.bfloat16, device="cuda")
+    _lib.call("lex_conv3d_pack_weights", _lib.ptr(w), c, c, 0, _lib.ptr(wp), _lib.stream())
+    out = [torch.zeros(n, c, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    for t, y in zip((x, off), out):
+        _lib.call("lex_conv3d_bf16_fwd", nx, ny, nz, c, c, _lib.ptr(t), _lib.ptr(wp), _lib.ptr(b), 1, 0, _lib.ptr(y),
+                  None, None, _lib.stream())
+    assert torch.equal(*out)
