@@ -489,11 +489,13 @@ __global__ void k_set_w_bc(Dims d, float* __restrict__ w) {
 }
 
 // x / r from the correctly rounded reciprocal ir of r: the product and one residual
-// correction, which is the correctly rounded quotient where nothing under- or overflows
-// (three operations instead of the ten of an IEEE division; r is a density).
+// correction, which is the correctly rounded quotient where nothing underflows.  Of an
+// infinite x, an infinite r or an overflow the residual is NaN; the product then has the
+// value that the division would give.  Five operations instead of the ten of an IEEE
+// division; r is a density.
 __device__ __forceinline__ float quotient(float x, float r, float ir) {
-  const float q = x * ir;
-  return fmaf(fmaf(-q, r, x), ir, q);
+  const float q = x * ir, y = fmaf(fmaf(-q, r, x), ir, q);
+  return y == y ? y : q;
 }
 
 // k_acoustic_m: one acoustic substep with each thread marching kAX cells along x: the x-face

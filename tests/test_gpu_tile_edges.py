@@ -70,6 +70,49 @@ def test_acoustic_substep_against_oracle(shape):
         check_fp32(from_dev(got), r64, r32, name)
 
 
+# an infinity in the middle of a lane's levels, at the last level of a wave and above the floor
+@pytest.mark.parametrize("shape,levels", [((9, 10, 24), (1, 12)), ((9, 10, 70), (5, 63, 64)),
+                                          ((9, 10, 140), (127, 128))], ids=str)
+def test_acoustic_substep_of_a_blown_up_state(shape, levels):
+    """Infinite w and u: the kernels give the infinities and NaNs of the oracle's IEEE arithmetic,
+    one substep at a time and two in one launch."""
+    import torch
+    from lex_amd import _lib
+    from oracle import lex_oracle as o
+    nx, ny, nz = shape
+    gr, phys, base = random_state(nx, ny, nz, seed=5, vel=2.0)
+    rng = np.random.default_rng(7)
+    th, u, v, w, p = (np.array(a, np.float32) for a in phys[:5])
+    ps = np.asarray(p + rng.normal(0, 1e-6, p.shape), np.float32)
+    for n, k in enumerate(levels):
+        w[6 - n, 6 + n, k + 1] = np.inf if n % 2 == 0 else -np.inf
+        u[7, 4, k + 1] = -np.inf
+    ru, rv, rw = (np.asarray(rng.normal(0, 1e-2, s), np.float32)
+                  for s in ((nx + 1, ny, nz), (nx, ny + 1, nz), (nx, ny, nz + 1)))
+    rho, pi0 = (np.asarray(base[q], np.float32) for q in (1, 3))
+    fixed = [to_dev(a) for a in (ps, ru, rv, rw, th)]
+    cols = [to_dev(a) for a in (rho[3, 3], pi0[3, 3])]
+    g = _lib.grid(nx, ny, nz, gr.dx, gr.dy, gr.dz)
+    f = lambda a: np.asarray(a, np.float64)  # noqa: E731
+
+    def call(name, state):
+        out = [torch.zeros_like(t) for t in state]
+        _lib.call(name, g, *[_lib.ptr(t) for t in (*cols, *state, *fixed)], 0.1, *[_lib.ptr(t) for t in out],
+                  _lib.stream())
+        return out
+
+    start = [to_dev(a) for a in (u, v, w, p)]
+    one = call("lex_acoustic_substep", start)
+    for n, got in ((1, one), (2, call("lex_acoustic_substep", one)), (2, call("lex_acoustic_substep_pair", start))):
+        with np.errstate(invalid="ignore"):
+            ref = o.sound_rk_step(f(u), f(v), f(w), f(pi0), f(p), f(ps), f(ru), f(rv), f(rw), f(th), f(rho), n, 0.1, gr)
+        for name, a, b in zip("u v w p".split(), got, ref):
+            a = from_dev(a)
+            assert np.array_equal(np.isnan(a), np.isnan(b)), (name, n)
+            assert np.array_equal(a[np.isinf(b)], b[np.isinf(b)]) and np.isinf(b).sum() == np.isinf(a).sum(), (name, n)
+    assert torch.isinf(one[3]).any()
+
+
 # one and two levels per lane, columns of one wave and of two, full and partial strips of
 # rows, marches of one and of several cells, the last one shorter
 @pytest.mark.parametrize("shape", [(6, 6, 24), (7, 13, 64), (100, 13, 40), (17, 9, 65), (33, 21, 128), (9, 7, 129),
