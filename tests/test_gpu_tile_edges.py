@@ -151,9 +151,10 @@ def test_smagorinsky_marches_equal_routine_chain(shape):
 
 
 # one and two levels per lane, the smallest and the fullest columns of each, one level left
-# over, marches of one and of several cells
-@pytest.mark.parametrize("shape", [(8, 9, 6), (17, 9, 64), (9, 7, 65), (9, 8, 127), (12, 11, 128), (161, 160, 33)],
-                         ids=str)
+# over, marches of one and of several cells; above 128 levels the workgroup-per-column form with
+# three and four waves, partly filled and full
+@pytest.mark.parametrize("shape", [(8, 9, 6), (17, 9, 64), (9, 7, 65), (9, 8, 127), (12, 11, 128), (161, 160, 33),
+                                   (8, 9, 129), (7, 10, 192), (6, 7, 193), (9, 8, 256)], ids=str)
 def test_implicit_substep_against_oracle(shape):
     """One vertically implicit substep against the FP64 oracle (a Thomas solve there); error
     within 8x the FP32 oracle's own, as for the other operators."""
