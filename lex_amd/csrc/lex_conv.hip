@@ -20,6 +20,9 @@ namespace lex {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// the same in memory at any element's address: callers' buffers are views as they come
+typedef bf16x4 bf16x4_any __attribute__((aligned(2)));
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
 
 constexpr int CTX = 4, CTY = 4, CTZ = 16;  // output tile of one workgroup (4 waves)
 constexpr int HX = CTX + 2, HY = CTY + 2, HZ = CTZ + 2;
@@ -454,7 +457,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3_rows(int nx, int ny, int nz, i
     bf16x4 res[WX][RTY];
     if constexpr (GGRAD) {
       rows([&](int a, int b, long c0) {
-        const f32x4 pa = *(const f32x4*)(pre + c0 * COUT + ch);
+        const f32x4 pa = *(const f32x4_any*)(pre + c0 * COUT + ch);
 #pragma unroll
         for (int i = 0; i < 4; ++i)   // padded channels: +0
           res[a][b][i] = (__bf16)(ch + i < cout_real ? acc[a][b][i] * gelu_t_grad(pa[i]) : 0.f);
@@ -470,21 +473,21 @@ __global__ __launch_bounds__(256, 2) void k_conv3_rows(int nx, int ny, int nz, i
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's part of the next planes
     rows([&](int a, int b, long c0) {
       const f32x4 v = acc[a][b];
-      if (!GGRAD && pre) *(f32x4*)(pre + c0 * COUT + ch) = v;
+      if (!GGRAD && pre) *(f32x4_any*)(pre + c0 * COUT + ch) = v;
       if constexpr (F32) {
         float* o = Yf + c0 * cout_real + ch;
         f32x4 r;
 #pragma unroll
         for (int i = 0; i < 4; ++i) r[i] = GELU ? gelu_t(v[i]) : v[i];
         if (cout_real == COUT) {
-          *(f32x4*)o = r;
+          *(f32x4_any*)o = r;
         } else {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
             if (ch + i < cout_real) o[i] = r[i];
         }
       } else {
-        *(bf16x4*)(Y + c0 * COUT + ch) = res[a][b];
+        *(bf16x4_any*)(Y + c0 * COUT + ch) = res[a][b];
       }
     });
   }

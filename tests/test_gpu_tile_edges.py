@@ -286,3 +286,46 @@ def test_conv_of_an_unaligned_view():
         _lib.call("lex_conv3d_bf16_fwd", nx, ny, nz, c, c, _lib.ptr(t), _lib.ptr(wp), _lib.ptr(b), 1, 0, _lib.ptr(y),
                   None, None, _lib.stream())
     assert torch.equal(*out)
+
+
+@pytest.mark.parametrize("cin,cout", [(16, 32), (32, 32), (32, 16), (16, 5)])
+def test_conv_with_unaligned_outputs(cin, cout):
+    """Outputs, pre-activations and the pre-activations that the data gradient reads, one element
+    off a 16-byte boundary: the bits of aligned buffers, and nothing beside them."""
+    import torch
+    from lex_amd import _lib
+    nx, ny, nz = 6, 7, 18
+    n, cop = nx * ny * nz, 16 * ((cout + 15) // 16)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn(n * cin, device="cuda", generator=gen).to(torch.bfloat16)
+    w, b = torch.randn(27, cin, cout, device="cuda", generator=gen), torch.randn(cop, device="cuda", generator=gen)
+    wp = torch.empty(cop * 28 * cin, dtype=torch.bfloat16, device="cuda")
+    _lib.call("lex_conv3d_pack_weights", _lib.ptr(w), cin, cout, 0, _lib.ptr(wp), _lib.stream())
+
+    def buf(count, dtype, off, fill=-7.0):
+        t = torch.full((count + off + 8,), fill, dtype=dtype, device="cuda")
+        assert t.data_ptr() % 16 == 0
+        return t, t[off:off + count]
+
+    def run(off):
+        whole, out = [], []
+        for c, dt in ((cop, torch.bfloat16), (cop, torch.float32), (cout, torch.float32)):
+            t, v = buf(n * c, dt, off)
+            whole.append(t)
+            out.append(v)
+        y, pre, yf = (_lib.ptr(v) for v in out)
+        args = (nx, ny, nz, cin, cout, _lib.ptr(x), _lib.ptr(wp), _lib.ptr(b))
+        _lib.call("lex_conv3d_bf16_fwd", *args, 1, 0, y, None, pre, _lib.stream())
+        _lib.call("lex_conv3d_bf16_fwd", *args, 1, 1, None, yf, None, _lib.stream())
+        if cop == 32:   # the same products as a data gradient, times the GELU's derivative at pre
+            t, v = buf(n * cop, torch.bfloat16, off)
+            whole.append(t)
+            out.append(v)
+            _lib.call("lex_conv3d_bf16_bwd_data_gelu", nx, ny, nz, cout, cin, _lib.ptr(x), _lib.ptr(wp), _lib.ptr(b),
+                      pre, _lib.ptr(v), _lib.stream())
+        for t, v in zip(whole, out):
+            assert bool((t[:off] == -7.0).all()) and bool((t[off + v.numel():] == -7.0).all())
+        return out
+
+    for a, c in zip(run(0), run(1)):
+        assert c.data_ptr() % 16 in (2, 4) and torch.equal(a, c)
