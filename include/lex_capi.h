@@ -346,8 +346,9 @@ int lex_rk3_step_vjp_taped(const lex_grid_t* g, const lex_step_opts_t* o, const 
  * W[kx*9 + ky*3 + kz][cin][cout] (flax's (3,3,3,in,out) kernel) packed to BF16 by
  * lex_conv3d_pack_weights (flip = 1 packs the transposed convolution of the data
  * gradient).  Accumulation is FP32.  Channels 1..64 (padded to 16, 32 or 64); the weight
- * gradient takes 1..32.  y, yf, pre, dx and g_pre_in need no more than their element's
- * alignment. */
+ * gradient takes 1..32.  No buffer but the packed weights (16 bytes) needs more than its
+ * element's alignment; the forward and the data gradients are slower with an x or g_pre off
+ * a 16-byte boundary, and allocate nothing. */
 size_t lex_conv3d_packed_weight_bytes(int cin, int cout, int flip);
 int lex_conv3d_pack_weights(const float* w, int cin, int cout, int flip, void* wp, void* stream);
 /* y = gelu?(conv(x) + bias): BF16 y (padded cout) or FP32 yf (cout channels); pre

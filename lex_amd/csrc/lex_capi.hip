@@ -1087,8 +1087,9 @@ void launch_fwd(int nx, int ny, int nz, const void* x, const void* wp, const flo
 #define LEX_ROWS(MD)                                                                                          \
   if ((mode & 15) == MD) {                                                                                    \
     const int run = conv_run(nx, tz * ty, conv_rows_resident<CI, CO, MD>());                                  \
-    hipLaunchKernelGGL((k_conv3_rows<CI, CO, MD>), dim3(tz, ty, (nx + run - 1) / run), dim3(256), 0, st, nx, ny, nz, \
-                       run, (const __bf16*)x, (const __bf16*)wp, bias, cout_real, (__bf16*)y, yf, pre);        \
+    const auto kernel = ((uintptr_t)x & 15) == 0 ? k_conv3_rows<CI, CO, MD, true> : k_conv3_rows<CI, CO, MD, false>; \
+    hipLaunchKernelGGL(kernel, dim3(tz, ty, (nx + run - 1) / run), dim3(256), 0, st, nx, ny, nz, run,          \
+                       (const __bf16*)x, (const __bf16*)wp, bias, cout_real, (__bf16*)y, yf, pre);             \
     return;                                                                                                   \
   }
     LEX_ROWS(0) LEX_ROWS(1) LEX_ROWS(2) LEX_ROWS(3) LEX_ROWS(4) LEX_ROWS(5) LEX_ROWS(6) LEX_ROWS(7)
@@ -1135,15 +1136,6 @@ static int conv_fwd(const char* name, int nx, int ny, int nz, int cin, int cout,
   // the GELU-gradient epilogue (mode 8) exists for 32 output channels in the marching kernel only
   if ((mode & 8) && (mode != 8 || cip > 32 || cop != 32 || !pre))
     return fail(-1, "%s: the fused GELU gradient needs <= 32 input and 17..32 output channels", name);
-  // the march copies 16-byte chunks of x into LDS: a view that starts elsewhere is moved first
-  SlotScratch sc;
-  if (((uintptr_t)x & 15) != 0 && cip <= 32 && cop <= 32) {
-    const size_t bytes = (size_t)nx * ny * nz * cip * 2;
-    if (sc.take(bytes, st) != hipSuccess) return fail(-4, "%s: no device memory for an aligned copy of x", name);
-    if (hipMemcpyAsync(sc.p, x, bytes, hipMemcpyDeviceToDevice, st) != hipSuccess)
-      return fail(-3, "%s: copying x failed", name);
-    x = sc.p;
-  }
 #define LEX_FWD(CI, CO) \
   if (cip == CI && cop == CO) { launch_fwd<CI, CO>(nx, ny, nz, x, wp, bias, mode, cout, y, yf, pre, st); return check_launch(name); }
   LEX_FWD(16, 16) LEX_FWD(16, 32) LEX_FWD(16, 64)

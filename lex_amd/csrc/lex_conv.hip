@@ -21,6 +21,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 // the same in memory at any element's address: callers' buffers are views as they come
+typedef bf16x8 bf16x8_any __attribute__((aligned(2)));
 typedef bf16x4 bf16x4_any __attribute__((aligned(2)));
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
 
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(256) void k_conv3_fwd(int nx, int ny, int nz, const
     }
     bf16x8 v;
     if (gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz) {
-      v = *(const bf16x8*)(X + (((long)gx * ny + gy) * nz + gz) * CIN + 8 * g);
+      v = *(const bf16x8_any*)(X + (((long)gx * ny + gy) * nz + gz) * CIN + 8 * g);
     } else {
       for (int j = 0; j < 8; ++j) v[j] = (__bf16)0.0f;
     }
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(256) void k_conv3_fwd32(int nx, int ny, int nz, con
     }
     bf16x8 v;
     if (gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz) {
-      v = *(const bf16x8*)(X + (((long)gx * ny + gy) * nz + gz) * CIN + 8 * g);
+      v = *(const bf16x8_any*)(X + (((long)gx * ny + gy) * nz + gz) * CIN + 8 * g);
     } else {
       for (int j = 0; j < 8; ++j) v[j] = (__bf16)0.0f;
     }
@@ -306,12 +307,15 @@ __global__ __launch_bounds__(256) void k_conv3_fwd32(int nx, int ny, int nz, con
 // Y), bit 2 periodic x and y, bit 3 GELU gradient: `pre` is read (the FP32 pre-activation of
 // the layer below, COUT channels) and Y = BF16((acc + bias) * gelu'(pre)), the data gradient
 // and the k_gelu_bwd pass after it in one (bits 0-2 clear).
+// ALIGNED: X starts at a 16-byte boundary, as the copies into LDS need; else the planes go
+// through registers (240 x 240 x 120, 32 -> 32: 366 and 498 us; moving such an X to an
+// aligned scratch copy first took 630 and memory that a caller may not have).
 constexpr int RSX = 4, RTY = 4, RTZ = 16;   // planes per step; rows and cells of a column
 constexpr int RRING = 2 * RSX + 2;          // halo planes in LDS
 
 __device__ const unsigned k_zero_chunk[4] __attribute__((aligned(16))) = {0, 0, 0, 0};
 
-template <int CIN, int COUT, int MODE>
+template <int CIN, int COUT, int MODE, bool ALIGNED>
 __global__ __launch_bounds__(256, 2) void k_conv3_rows(int nx, int ny, int nz, int run, const __bf16* __restrict__ X,
                                                        const __bf16* __restrict__ Wp, const float* __restrict__ bias,
                                                        int cout_real, __bf16* __restrict__ Y, float* __restrict__ Yf,
@@ -362,9 +366,14 @@ __global__ __launch_bounds__(256, 2) void k_conv3_rows(int nx, int ny, int nz, i
     return 8 * ((c % NCH) ^ swz(hz));
   };
   auto put = [&](int q, int slot, const void* src) {
-    if (PLC % 64 == 0 || (q % GP) * 64 + l < PLC)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)(ring + slot * PLANE + (q % GP) * 512), 16, 0, 0);
+    if (PLC % 64 == 0 || (q % GP) * 64 + l < PLC) {
+      if constexpr (ALIGNED)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                         (__attribute__((address_space(3))) void*)(ring + slot * PLANE + (q % GP) * 512),
+                                         16, 0, 0);
+      else
+        *(bf16x8*)(ring + slot * PLANE + (q % GP) * 512 + 8 * l) = *(const bf16x8_any*)src;
+    }
   };
   // byte offsets of the lane's chunks of a step's planes from (plane, y0 - 1, z0 - 1)
   uint32_t off[NPF];
@@ -517,7 +526,7 @@ inline int conv_rows_resident() {
     int dev = 0, ncu = 0, per = 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_conv3_rows<CIN, COUT, MODE>, 256, 0);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_conv3_rows<CIN, COUT, MODE, true>, 256, 0);
     return (ncu > 0 ? ncu : 256) * (per > 0 ? per : 1);
   }();
   return resident;
@@ -597,7 +606,7 @@ __global__ __launch_bounds__(512) void k_conv3_wgrad(int nx, int ny, int nz, con
   auto ld = [&](const __bf16* f, int ch, int x, int y, int z, int c0) {
     bf16x8 v = {};
     if (x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz)
-      v = *(const bf16x8*)(f + (((long)x * ny + y) * nz + z) * ch + c0);
+      v = *(const bf16x8_any*)(f + (((long)x * ny + y) * nz + z) * ch + c0);
     return v;
   };
   auto fetch = [&](int tile) {

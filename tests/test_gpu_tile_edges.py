@@ -329,3 +329,45 @@ def test_conv_with_unaligned_outputs(cin, cout):
 
     for a, c in zip(run(0), run(1)):
         assert c.data_ptr() % 16 in (2, 4) and torch.equal(a, c)
+
+
+@pytest.mark.parametrize("cin,cout,circular", [(16, 16, False), (16, 32, True), (32, 16, True), (32, 32, False)])
+def test_conv_of_an_unaligned_view_takes_no_memory(cin, cout, circular):
+    """An input off a 16-byte boundary, whole and partial tiles, all outputs: the aligned input's
+    bits, and the device's free memory as before (the calls may run where none can be taken)."""
+    import torch
+    from lex_amd import _lib
+    nx, ny, nz = 70, 67, 275
+    n = nx * ny * nz
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    buf = torch.empty(n * cin + 8, dtype=torch.bfloat16, device="cuda")
+    x = torch.randn(n * cin, device="cuda", generator=gen).to(torch.bfloat16)
+    w, b = torch.randn(27, cin, cout, device="cuda", generator=gen), torch.randn(cout, device="cuda", generator=gen)
+    wp = torch.empty(cout * 28 * cin, dtype=torch.bfloat16, device="cuda")
+    _lib.call("lex_conv3d_pack_weights", _lib.ptr(w), cin, cout, 0, _lib.ptr(wp), _lib.stream())
+    entry = "lex_conv3d_bf16_fwd_circular" if circular else "lex_conv3d_bf16_fwd"
+
+    def outputs():
+        return [torch.full((n * cout,), -7.0, dtype=t, device="cuda")
+                for t in (torch.bfloat16, torch.float32, torch.float32, torch.bfloat16)]
+
+    def run(v, out):
+        y, pre, yf, dx = (_lib.ptr(t) for t in out)
+        args = (nx, ny, nz, cin, cout, _lib.ptr(v), _lib.ptr(wp), _lib.ptr(b))
+        _lib.call(entry, *args, 1, 0, y, None, pre, _lib.stream())
+        _lib.call(entry, *args, 0, 1, None, yf, None, _lib.stream())
+        if cout == 32:
+            _lib.call("lex_conv3d_bf16_bwd_data_gelu", nx, ny, nz, cout, cin, *args[5:], pre, dx, _lib.stream())
+        torch.cuda.synchronize()
+
+    want, got = outputs(), outputs()
+    run(x, want)
+    for off in (1, 4):
+        v = buf[off:off + n * cin].copy_(x)
+        assert v.data_ptr() % 16 == 2 * off
+        free = torch.cuda.mem_get_info()[0]
+        run(v, got)
+        assert free - torch.cuda.mem_get_info()[0] < n * cin   # half of x
+        for a, c in zip(got, want):
+            assert torch.equal(a, c)
+            a.fill_(-7.0)
