@@ -298,7 +298,7 @@ __global__ __launch_bounds__(256) void k_conv3_fwd32(int nx, int ny, int nz, con
 // input channels (365 us: spills).
 //
 // K: for 32 input channels one step per tap; for 16 a step is two z taps, (-1, 0) and (+1, -),
-// lanes 0-31 reading the first and 32-63 the second.  Cells lie unpadded in LDS; for 32
+// lanes 0-31 reading the first and 32-63 the second (zeros where there is none).  Cells lie unpadded in LDS; for 32
 // channels the upper and lower 32 bytes of a cell change places where bit 2 of its z position
 // is set, which puts the 16 lanes that an operand read serves at a time (0-3, 12-15, 20-27 and
 // 4-11, 16-19, 28-31 of each half wave) on all 64 banks.
@@ -330,7 +330,11 @@ __global__ __launch_bounds__(256, 2) void k_conv3_rows(int nx, int ny, int nz, i
   constexpr int NPF = (RSX * GP + 3) / 4;                       // accesses per wave and step
   constexpr int NZG = CIN == 32 ? 3 : 2;                        // K steps per (x, y) tap
   constexpr int KROW = ConvSteps<CIN>::NSTEP * 32;              // packed weights of one output channel
-  __shared__ __attribute__((aligned(16))) __bf16 ring[RRING * PLANE];
+  // 16 input channels: zeros for the lanes of the second K step that have no tap, which read
+  // them at the offset of every row (a zero weight times an infinity would be NaN)
+  constexpr int ZEROS = CIN == 16 ? (GY - 1) * GZ * CIN + 8 : 0;
+  __shared__ __attribute__((aligned(16))) __bf16 ring[RRING * PLANE + ZEROS];
+  for (int e = threadIdx.x; e < ZEROS; e += 256) ring[RRING * PLANE + e] = (__bf16)0.0f;
   const TileId tb = xcd_tile();
   const int z0 = tb.x * RTZ, y0 = tb.y * RTY, xa = tb.z * run, xb = min(xa + run, nx);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, m = l & 15, g = l >> 4;
@@ -428,7 +432,9 @@ __global__ __launch_bounds__(256, 2) void k_conv3_rows(int nx, int ny, int nz, i
     bf16x8 f[2][GY];
     auto read = [&](int gi, bf16x8(&d)[GY]) {
       const int s = slot + xw + gi / NZG;
-      const __bf16* r = ring + (s >= RRING ? s - RRING : s) * PLANE + lb[gi % NZG];
+      int e = (s >= RRING ? s - RRING : s) * PLANE + lb[gi % NZG];
+      if (CIN == 16 && gi % NZG == 1 && g >= 2) e = RRING * PLANE;
+      const __bf16* r = ring + e;
 #pragma unroll
       for (int y = 0; y < GY; ++y) d[y] = *(const bf16x8*)(r + y * GZ * CIN);
     };

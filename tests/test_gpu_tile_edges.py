@@ -371,3 +371,24 @@ def test_conv_of_an_unaligned_view_takes_no_memory(cin, cout, circular):
         for a, c in zip(got, want):
             assert torch.equal(a, c)
             a.fill_(-7.0)
+
+
+@pytest.mark.parametrize("cin,cout", [(5, 32), (16, 16), (16, 32), (32, 32), (32, 5)])
+def test_conv_of_an_infinite_cell(cin, cout):
+    """An infinite activation gives an infinity of the weight's sign at each of the 27 outputs that
+    it reaches, and leaves the others as they are."""
+    import torch
+    from lex_amd import sgs_net as sn
+    shape = (9, 10, 35)
+    gen = torch.Generator().manual_seed(3)
+    x = torch.randn(*shape, cin, generator=gen)
+    w, b = torch.randn(27, cin, cout, generator=gen), torch.randn(cout, generator=gen)
+    run = lambda t: sn.conv3d_fwd(sn.to_bf16_channels_last(t.cuda()), shape, w.cuda(), b.cuda(), gelu=False,  # noqa: E731
+                                  out_fp32=True)[0].cpu().view(*shape, cout)
+    want = run(x)
+    for cell, c, v in (((4, 5, 17), 0, float("inf")), ((1, 7, 30), cin - 1, -float("inf"))):
+        x[(*cell, c)] = v
+        for tap in range(27):
+            o = [a - d + 1 for a, d in zip(cell, (tap // 9, tap // 3 % 3, tap % 3))]
+            want[tuple(o)] = v * w[tap, c].sign()
+    assert torch.equal(run(x), want)
