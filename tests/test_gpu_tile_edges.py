@@ -217,10 +217,12 @@ def test_bicgstab_first_iterations_against_oracle(shape):
 
 
 # runs shorter than a step, of one step, and long enough to go round the ring of planes; one
-# and several rows and z tiles with and without a remainder; 16 and 32 channels either side
+# and several rows and z tiles with and without a remainder; periods of two and three cells,
+# which a step's planes and rows run round more than once; 16 and 32 channels either side
 @pytest.mark.parametrize("circular", [False, True])
 @pytest.mark.parametrize("cin,cout", [(5, 32), (32, 32), (32, 5), (16, 16)])
-@pytest.mark.parametrize("shape", [(4, 4, 16), (7, 5, 17), (46, 9, 35), (97, 66, 33)], ids=str)
+@pytest.mark.parametrize("shape", [(4, 4, 16), (7, 5, 17), (46, 9, 35), (97, 66, 33), (2, 3, 18), (3, 2, 16),
+                                   (2, 2, 3), (2, 21, 40), (19, 3, 40)], ids=str)
 def test_convolution_march(shape, cin, cout, circular):
     """One convolution against torch conv3d in float64 on the same BF16 operands: FP32 sums of
     27 cin products, 1e-5 as for the other sizes; the BF16 output is its rounding (2^-8)."""
