@@ -1083,12 +1083,12 @@ template <int CI, int CO>
 void launch_fwd(int nx, int ny, int nz, const void* x, const void* wp, const float* bias, int mode, int cout_real,
                 void* y, float* yf, float* pre, hipStream_t st) {
   if constexpr (CI <= 32 && CO <= 32) {   // weights in registers, march along x
-    const int tz = (nz + RTZ - 1) / RTZ, ty = (ny + RTY - 1) / RTY;
+    const long cols = (long)((nz + RTZ - 1) / RTZ) * ((ny + RTY - 1) / RTY);
 #define LEX_ROWS(MD)                                                                                          \
   if ((mode & 15) == MD) {                                                                                    \
-    const int run = conv_run(nx, tz * ty, conv_rows_resident<CI, CO, MD>());                                  \
+    const int run = conv_run(nx, cols, conv_rows_resident<CI, CO, MD>());                                  \
     const auto kernel = ((uintptr_t)x & 15) == 0 ? k_conv3_rows<CI, CO, MD, true> : k_conv3_rows<CI, CO, MD, false>; \
-    hipLaunchKernelGGL(kernel, dim3(tz, ty, (nx + run - 1) / run), dim3(256), 0, st, nx, ny, nz, run,          \
+    hipLaunchKernelGGL(kernel, conv_rows_grid(nx, ny, nz, run), dim3(256), 0, st, nx, ny, nz, run,             \
                        (const __bf16*)x, (const __bf16*)wp, bias, cout_real, (__bf16*)y, yf, pre);             \
     return;                                                                                                   \
   }

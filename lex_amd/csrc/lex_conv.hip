@@ -335,8 +335,13 @@ __global__ __launch_bounds__(256, 2) void k_conv3_rows(int nx, int ny, int nz, i
   constexpr int ZEROS = CIN == 16 ? (GY - 1) * GZ * CIN + 8 : 0;
   __shared__ __attribute__((aligned(16))) __bf16 ring[RRING * PLANE + ZEROS];
   for (int e = threadIdx.x; e < ZEROS; e += 256) ring[RRING * PLANE + e] = (__bf16)0.0f;
+  // workgroups: z tile, then row, then run of planes (conv_rows_grid)
   const TileId tb = xcd_tile();
-  const int z0 = tb.x * RTZ, y0 = tb.y * RTY, xa = tb.z * run, xb = min(xa + run, nx);
+  const unsigned tz = (nz + RTZ - 1) / RTZ, ty = (ny + RTY - 1) / RTY;
+  const unsigned id = tb.x + gridDim.x * tb.y, col = id / tz, part = col / ty;
+  const int z0 = (int)(id - col * tz) * RTZ, y0 = (int)(col - part * ty) * RTY;
+  const int xa = (int)part * run, xb = min(xa + run, nx);
+  if (xa >= nx) return;   // past the last workgroup of a grid in two dimensions
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, m = l & 15, g = l >> 4;
   const int ch = (w % NH) * 16 + 4 * g, xw = (w / NH) * WX;     // first output channel of the lane; first plane
   auto swz = [](int z) { return CIN == 32 ? (z >> 1) & 2 : 0; };
@@ -510,12 +515,12 @@ __global__ __launch_bounds__(256, 2) void k_conv3_rows(int nx, int ny, int nz, i
 
 // x planes per workgroup: whole steps, so many that the workgroups fill the device evenly.
 // A run costs its planes and about one step more (the first planes, the weights).
-inline int conv_run(int nx, int cols, int resident) {
+inline int conv_run(int nx, long cols, int resident) {
   int best = 0;
   double cost = 0.0;
   for (int runs = 1; runs <= (nx + RSX - 1) / RSX && runs <= 256; ++runs) {
     const int len = ((nx + runs - 1) / runs + RSX - 1) / RSX * RSX;
-    const long n = (long)cols * ((nx + len - 1) / len);
+    const long n = cols * ((nx + len - 1) / len);
     const double c = (double)((n + resident - 1) / resident) * (len + RSX);
     if (best == 0 || c < cost) {
       best = len;
@@ -523,6 +528,14 @@ inline int conv_run(int nx, int cols, int resident) {
     }
   }
   return best;
+}
+
+// One dimension up to 2^20 workgroups, as rows or z tiles in the grid's second or third would
+// bound them at 2^16; more in rows of 2^20.
+inline dim3 conv_rows_grid(int nx, int ny, int nz, int run) {
+  const long n = (long)((nz + RTZ - 1) / RTZ) * ((ny + RTY - 1) / RTY) * ((nx + run - 1) / run);
+  const long rows = (n + (1L << 20) - 1) >> 20;
+  return dim3((unsigned)(rows > 1 ? 1L << 20 : n), (unsigned)rows);
 }
 
 // workgroups the device holds at once (occupancy from the runtime)

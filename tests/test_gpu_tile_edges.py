@@ -394,3 +394,17 @@ def test_conv_of_an_infinite_cell(cin, cout):
             o = [a - d + 1 for a, d in zip(cell, (tap // 9, tap // 3 % 3, tap % 3))]
             want[tuple(o)] = v * w[tap, c].sign()
     assert torch.equal(run(x), want)
+
+
+@pytest.mark.parametrize("shape", [(1, 262153, 1), (262153, 2, 2), (2, 1, 1048601)], ids=str)
+def test_conv_of_a_long_grid(shape):
+    """More rows than a launch has in its second dimension, and as long in x and z."""
+    import torch
+    from lex_amd import sgs_net as sn
+    gen = torch.Generator().manual_seed(3)
+    x, w = torch.randn(*shape, 5, generator=gen), torch.randn(27, 5, 5, generator=gen)
+    xb, wb = x.bfloat16().double().permute(3, 0, 1, 2)[None], w.bfloat16().double().view(3, 3, 3, 5, 5)
+    ref = torch.nn.functional.conv3d(xb, wb.permute(4, 3, 0, 1, 2), padding=1)[0].permute(1, 2, 3, 0)
+    got, _ = sn.conv3d_fwd(sn.to_bf16_channels_last(x.cuda()), shape, w.cuda(), torch.zeros(5, device="cuda"),
+                           gelu=False, out_fp32=True)
+    assert float((got.cpu().double().view(*shape, 5) - ref).norm() / ref.norm()) < 1e-5
