@@ -731,7 +731,7 @@ template <int V, bool MZ, int ROWS>
 inline void launch_acoustic2_v(const Dims& d, const AcousticArgs& a, hipStream_t st) {
   constexpr int kLanes = MZ ? 128 : 64;
   const int strips = (d.ny + ROWS - 3) / (ROWS - 2);
-  const int parts = std::max(1, std::min(d.nx, (V == 1 ? 512 : 256) / strips));
+  const int parts = std::max(1, std::min(d.nx, device_cus() * (V == 1 ? 2 : 1) / strips));
   const int ax = (d.nx + parts - 1) / parts;
   const dim3 g(strips, (d.nx + ax - 1) / ax), b(kLanes, ROWS);
   const size_t lds = (size_t)2 * ROWS * kLanes * V * sizeof(float);

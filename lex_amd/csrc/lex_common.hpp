@@ -10,8 +10,23 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <atomic>
 
 namespace lex {
+
+// CUs of the current device, for plans that fill it (256 of a whole chip; a partition has
+// fewer), kept per device index.
+inline int device_cus() {
+  static std::atomic<int> kept[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = kept[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+    kept[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
 
 // Physical constants: namelist_n_constants.py:64-75 (rounded to FP32 the way JAX
 // rounds weak Python scalars).

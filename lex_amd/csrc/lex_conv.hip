@@ -541,14 +541,12 @@ inline dim3 conv_rows_grid(int nx, int ny, int nz, int run) {
 // workgroups the device holds at once (occupancy from the runtime)
 template <int CIN, int COUT, int MODE>
 inline int conv_rows_resident() {
-  static const int resident = [] {
-    int dev = 0, ncu = 0, per = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  static const int per_cu = [] {
+    int per = 0;
     (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_conv3_rows<CIN, COUT, MODE, true>, 256, 0);
-    return (ncu > 0 ? ncu : 256) * (per > 0 ? per : 1);
+    return per > 0 ? per : 1;
   }();
-  return resident;
+  return device_cus() * per_cu;
 }
 
 // Weight gradient: dW[tap][c][n] += sum_p X[p + o(tap)][c] * G[p][n] over the cells of

@@ -702,7 +702,7 @@ inline size_t stage_lds(const Dims& d) {   // the w piece's, the largest
 // scalars (16) 4034, 3190, 3085, 3059, 3104.  Within the bound the tiles are made even.
 inline int stage_ax(const Dims& d, int pieces) {
   const int threads = 64 * ((d.nz + 63) / 64) * kFTY;
-  const int slots = 256 * (24 * 64 / threads);   // 24 waves per CU at 80 VGPRs
+  const int slots = device_cus() * (24 * 64 / threads);   // 24 waves per CU at 80 VGPRs
   const double n = (double)pieces * ((d.ny + kFTY - 1) / kFTY) * d.nx;
   const int ax = std::min(kFTX, std::max(1, (int)lround(sqrt(2.0 * n / slots))));
   const int tiles = (d.nx + ax - 1) / ax;

@@ -471,7 +471,7 @@ inline size_t smag_fused_lds(const Dims& d, bool aniso) {
 inline int smag_fused_ax(const Dims& d) {
   const int ty = smag_fused_rows(d) - 2, strips = (d.ny + ty - 1) / ty;
   const int threads = 64 * ((d.nz + 63) / 64) * smag_fused_rows(d);
-  const int parts = std::max(1, 256 * (1536 / threads) / strips);
+  const int parts = std::max(1, device_cus() * (1536 / threads) / strips);
   return std::min(16, (d.nx + parts - 1) / parts);
 }
 inline dim3 smag_fused_grid(const Dims& d) {
