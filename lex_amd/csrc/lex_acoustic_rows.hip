@@ -325,40 +325,110 @@ __global__ void __launch_bounds__(256) k_acoustic(Dims d, const float* __restric
   }
 }
 
+// The same substep with a thread per cell, which takes every face twice but loads nothing that
+// depends on anything else: for columns of more than two waves.
+__global__ void __launch_bounds__(256) k_acoustic_cells(Dims d, const float* __restrict__ rc,
+                                                        const float* __restrict__ pi0c, const float* __restrict__ u,
+                                                        const float* __restrict__ v, const float* __restrict__ w,
+                                                        const float* __restrict__ p, const float* __restrict__ ps,
+                                                        const float* __restrict__ ru, const float* __restrict__ rv,
+                                                        const float* __restrict__ rw, const float* __restrict__ tr,
+                                                        float* __restrict__ uo, float* __restrict__ vo,
+                                                        float* __restrict__ wo, float* __restrict__ po, float dts) {
+#pragma clang fp contract(off)
+  const TileId tb = xcd_tile();
+  const int k = tb.x * (int)blockDim.x + (int)threadIdx.x, j = tb.y * (int)blockDim.y + (int)threadIdx.y, i = tb.z;
+  if (k >= d.nz || j >= d.ny) return;
+  const int I = i + 3, J = j + 3, K = k + 1;
+  const long c = ic(d, I, J, K), sx = d.sxc(), sy = d.syc();
+  const long cu = iu(d, I, J, K), cv = iv(d, I, J, K), cw = iw(d, I, J, K);
+  const long ou = ((long)i * d.ny + j) * d.nz + k, ov = ((long)i * (d.ny + 1) + j) * d.nz + k;
+  const long ow = ((long)i * d.ny + j) * (d.nz + 1) + k;
+  // every operand is loaded unconditionally (all indices are inside the arrays) so that the
+  // loads issue back to back; the surface and lid cases are selected afterwards
+  const float rcm = rc[K - 1], rcc = rc[K], rcp = rc[K + 1];
+  const float pim = pi0c[K - 1], pic = pi0c[K], pip = pi0c[K + 1];
+  const float u0 = u[cu], u1 = u[cu + d.sxu()], v0 = v[cv], v1 = v[cv + sy], w0 = w[cw], w1 = w[cw + 1];
+  const float ru0 = ru[ou], ru1 = ru[ou + (long)d.ny * d.nz], rv0 = rv[ov], rv1 = rv[ov + d.nz];
+  const float rw0 = rw[ow], rw1 = rw[ow + 1];
+  const float pc = p[c], pxm = p[c - sx], pxp = p[c + sx], pym = p[c - sy], pyp = p[c + sy], pzm = p[c - 1],
+              pzp = p[c + 1];
+  const float tc = tr[c], txm = tr[c - sx], txp = tr[c + sx], tym = tr[c - sy], typ = tr[c + sy], tzm = tr[c - 1],
+              tzp = tr[c + 1];
+  const float sc = ps[c], sxm = ps[c - sx], sxp = ps[c + sx], sym = ps[c - sy], syp = ps[c + sy], szm = ps[c - 1],
+              szp = ps[c + 1];
+  const bool floor_ = k == 0, lid = k == d.nz - 1;
+  const float h = (float)(-kCp * 0.5);
+  const float un0 = fmaf(fmaf(h * (tc + txm), (pc - pxm) * d.idx, ru0), dts, u0);
+  const float un1 = fmaf(fmaf(h * (txp + tc), (pxp - pc) * d.idx, ru1), dts, u1);
+  const float vn0 = fmaf(fmaf(h * (tc + tym), (pc - pym) * d.idy, rv0), dts, v0);
+  const float vn1 = fmaf(fmaf(h * (typ + tc), (pyp - pc) * d.idy, rv1), dts, v1);
+  const float wn0 = floor_ ? 0.0f : fmaf(h * (tc + tzm) * ((pc - pzm) * d.idz) + rw0, dts, w0);
+  const float wn1 = lid ? 0.0f : fmaf(h * (tzp + tc) * ((pzp - pc) * d.idz) + rw1, dts, w1);
+  const float div = fmaf(wn1 - wn0, d.idz, fmaf(vn1 - vn0, d.idy, (un1 - un0) * d.idx));
+  const float du = un1 * ((sxp - sc) * d.idx) + un0 * ((sc - sxm) * d.idx);
+  const float dv = vn1 * ((syp - sc) * d.idy) + vn0 * ((sc - sym) * d.idy);
+  const float wd0 = floor_ ? 0.0f : wn0 * fmaf(sc - szm, d.idz, (pic - pim) * d.idz);
+  const float wd1 = lid ? 0.0f : wn1 * fmaf(szp - sc, d.idz, (pip - pic) * d.idz);
+  const float z = fmaf(0.5f * wd0, 0.5f * (rcm + rcc), 0.5f * wd1 * (0.5f * (rcc + rcp))) / rcc;
+  const float advp = -(fmaf(0.5f, du, 0.5f * dv) + z);
+  const float dpdt = fmaf((float)(-kRd / kCv), (pic + sc) * div, advp);
+  store_c_fast(d, po, i, j, k, fmaf(1.1f * dpdt, dts, pc));
+  store_u_fast(d, uo, i, j, k, un0);
+  if (i == d.nx - 1) store_u(d, uo, d.nx, j, k, un1);
+  store_v_fast(d, vo, i, j, k, vn0);
+  if (j == d.ny - 1) store_v(d, vo, i, d.ny, k, vn1);
+  store_w_fast(d, wo, i, j, k, wn0);
+  if (lid) store_w(d, wo, i, j, d.nz, 0.0f);
+}
+
 struct AcousticArgs {
   const float *rc, *pi0, *u, *v, *w, *p, *ps, *ru, *rv, *rw, *tr;
   float *uo, *vo, *wo, *po;
   float dts;
 };
 
-template <int V>
+template <int V, bool MZ>
 inline void launch_acoustic_v(const Dims& d, const AcousticArgs& a, hipStream_t st) {
   const int chunks = (d.nz + 64 * V - 1) / (64 * V);
   // Cells per wave along x: the prologue of a longer march is shared, as long as the launch
-  // keeps some 16 waves on every SIMD.  us per substep at ax = 1, 2, 4, 6: 96x96x48 11.2,
-  // 12.6, 16.2, 19.5; 128x128x64 15.6, 16.8, 19.4, 19.9; 181x147x70 38.0, 32.6, 31.6, 33.7;
-  // 192x160x96 43.6, 38.8, 40.9, 39.8; 240x240x120 111, 99, 97, 97; 256x256x128 129, 115, 113, 110.
+  // has some 16 waves per SIMD, two rounds or more.  us per substep at ax = 1, 2, 3, 4, one
+  // level per lane: 128x128x64 15.6, 16.8, -, 19.4; 200x200x64 27.1, 27.1, 26.6, 27.1; 300x200x64
+  // 37.6, 35.8, 39.0, 41.2; 1000x60x64 38.7, 36.7, 40.0, 44.6; 512x300x64 139, 133, 131, 133; two:
+  // 128x96x96 20.2, 20.9, 19.9, -; 150x130x80 27.0, 25.3, 27.3, -; 192x160x96 43.6, 38.8, -, 40.9;
+  // 200x200x80 49.6, 43.2, 40.3, 43.5; 240x240x120 111, 99, -, 97; 256x256x128 129, 115, -, 113.
   const long waves = (long)d.nx * d.ny * chunks;
-  const int ax = (int)std::min(4L, std::max(1L, (waves + 8192) / 16384));
-  const dim3 g((d.ny + 3) / 4, (d.nx + ax - 1) / ax, chunks), b(64, 4, 1);
-  if (chunks == 1)
-    LEX_LAUNCH(KID_ACOUSTIC, (k_acoustic<V, false>), g, b, 0, st, d, a.rc, a.pi0, a.u, a.v, a.w, a.p, a.ps, a.ru, a.rv,
-               a.rw, a.tr, a.uo, a.vo, a.wo, a.po, a.dts, ax);
-  else
-    LEX_LAUNCH(KID_ACOUSTIC, (k_acoustic<V, true>), g, b, 0, st, d, a.rc, a.pi0, a.u, a.v, a.w, a.p, a.ps, a.ru, a.rv,
-               a.rw, a.tr, a.uo, a.vo, a.wo, a.po, a.dts, ax);
+  const int ax = V == 1 ? (int)std::min(2L, std::max(1L, (waves + 8192) / 16384))
+                        : (int)std::min(4L, std::max(1L, (waves + 14000) / 16384));
+  LEX_LAUNCH(KID_ACOUSTIC, (k_acoustic<V, MZ>), dim3((d.ny + 3) / 4, (d.nx + ax - 1) / ax, chunks), dim3(64, 4, 1), 0, st,
+             d, a.rc, a.pi0, a.u, a.v, a.w, a.p, a.ps, a.ru, a.rv, a.rw, a.tr, a.uo, a.vo, a.wo, a.po, a.dts, ax);
+}
+inline void launch_acoustic_cells(const Dims& d, const AcousticArgs& a, hipStream_t st) {
+  LEX_LAUNCH(KID_ACOUSTIC, k_acoustic_cells, dim3((d.nz + 63) / 64, (d.ny + 3) / 4, d.nx), dim3(64, 4, 1), 0, st, d, a.rc,
+             a.pi0, a.u, a.v, a.w, a.p, a.ps, a.ru, a.rv, a.rw, a.tr, a.uo, a.vo, a.wo, a.po, a.dts);
 }
 
 // One substep.  Two levels per lane where a column has more than one wave of them; us with
 // one and with two: 96x96x48 11.2 and 17.9, 128x128x64 15.6 and 26.6 (half the lanes idle);
-// 181x147x70 33.1 and 31.6, 240x240x120 120 and 97, 256x256x128 139 and 110.  The
-// cell-per-thread form took 13.9, 17.9, 35.8, 113 and 131; a copy of the thirteen fields of
-// 240x240x120 at 5 TB/s takes 72.
+// 181x147x70 33.1 and 31.6, 240x240x120 120 and 97, 256x256x128 139 and 110.  A thread per
+// cell took 13.9, 17.9, 35.8, 113 and 131; a copy of the thirteen fields of 240x240x120 at
+// 5 TB/s takes 72.
+// Above 128 levels a row of lanes leaves its last wave part empty, which costs as much as a
+// full one, and rows take longer chains of loads than cells: us with rows and cells,
+// 128x128x129 39 and 31, 192x160x160 91 and 66, 256x256x160 207 and 161, 192x160x300 160 and
+// 141, 256x256x384 422 and 365.  With both waves of two levels nearly full the rows win while
+// the chip is not, and again where memory bounds both: 64x64x224 16.4 and 17.5, 128x96x224 36
+// and 33, 128x128x256 48 and 44, 192x160x224 108 and 116, 256x256x256 230 and 254.
 inline void launch_acoustic(const Dims& d, const AcousticArgs& a, hipStream_t st) {
-  if (d.nz > 64)
-    launch_acoustic_v<2>(d, a, st);
+  const long cells = (long)d.nx * d.ny * d.nz;
+  if (d.nz <= 64)
+    launch_acoustic_v<1, false>(d, a, st);
+  else if (d.nz <= 128)
+    launch_acoustic_v<2, false>(d, a, st);
+  else if (d.nz > 192 && d.nz <= 256 && (cells < 1500000 || cells >= 5000000))
+    launch_acoustic_v<2, true>(d, a, st);
   else
-    launch_acoustic_v<1>(d, a, st);
+    launch_acoustic_cells(d, a, st);
 }
 
 // k_acoustic2: two consecutive substeps in one launch, bit for bit what two k_acoustic

@@ -38,9 +38,9 @@ def test_stage_tiles_equal_per_operator_kernels(shape, passive):
 
 
 # one and two levels per lane, columns of one wave and of several with one level left over,
-# even and odd nz, marches of one and of several cells
+# even and odd nz, marches of one and of several cells; a thread per cell above 128 levels
 @pytest.mark.parametrize("shape", [(8, 9, 24), (17, 9, 64), (9, 7, 65), (33, 18, 128), (6, 6, 129), (20, 21, 200),
-                                   (161, 120, 73)], ids=str)
+                                   (161, 120, 73), (9, 10, 192), (12, 6, 193), (90, 91, 250), (7, 8, 321)], ids=str)
 def test_acoustic_substep_against_oracle(shape):
     """One substep against the FP64 oracle, the input's ghosts not periodic images (an initial
     state's need not be); error within 8x the FP32 oracle's own, as for the other operators."""
@@ -72,7 +72,7 @@ def test_acoustic_substep_against_oracle(shape):
 
 # an infinity in the middle of a lane's levels, at the last level of a wave and above the floor
 @pytest.mark.parametrize("shape,levels", [((9, 10, 24), (1, 12)), ((9, 10, 70), (5, 63, 64)),
-                                          ((9, 10, 140), (127, 128))], ids=str)
+                                          ((9, 10, 140), (127, 128)), ((9, 10, 230), (127, 128))], ids=str)
 def test_acoustic_substep_of_a_blown_up_state(shape, levels):
     """Infinite w and u: the kernels give the infinities and NaNs of the oracle's IEEE arithmetic,
     one substep at a time and two in one launch."""
