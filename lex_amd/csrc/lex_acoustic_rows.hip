@@ -794,15 +794,26 @@ __global__ void __launch_bounds__(MAXT) k_acoustic2(Dims d, AcousticArgs a, int 
 inline bool acoustic2_ok(const Dims& d) { return d.nz <= 256; }
 
 // ROWS: two levels per lane need 142 to 160 VGPRs, three waves per SIMD, so one workgroup of
-// twelve waves fills a CU; with one level (87 VGPRs) two workgroups of eight.  The march is as
-// long as leaves every CU its workgroups once: a second, partly filled round costs more than
-// the two positions that a longer march saves.
+// twelve waves fills a CU; with one level (87 VGPRs) two workgroups of eight.  The march is the
+// one of 1 to 8 full rounds of workgroups that takes the fewest steps, a workgroup of ax cells
+// taking ax + 3.  One round is best while its strips divide the CUs; us with one round and with
+// this plan, 500x520x130 (131 strips) 2130 and 1082, 1024x1024x32 (171 of 512) 1587 and 869,
+// 300x1600x40 939 and 456, 512x512x100 620 and 540, 240x240x120 (24) 141 and 141.
 template <int V, bool MZ, int ROWS>
 inline void launch_acoustic2_v(const Dims& d, const AcousticArgs& a, hipStream_t st) {
   constexpr int kLanes = MZ ? 128 : 64;
   const int strips = (d.ny + ROWS - 3) / (ROWS - 2);
-  const int parts = std::max(1, std::min(d.nx, device_cus() * (V == 1 ? 2 : 1) / strips));
-  const int ax = (d.nx + parts - 1) / parts;
+  const long slots = (long)device_cus() * (V == 1 ? 2 : 1);
+  int ax = d.nx;
+  long least = 0;
+  for (int rounds = 1; rounds <= 8; ++rounds) {
+    const int parts = (int)std::max(1L, std::min((long)d.nx, rounds * slots / strips)), len = (d.nx + parts - 1) / parts;
+    const long n = (long)strips * ((d.nx + len - 1) / len), cost = (n + slots - 1) / slots * (len + 3);
+    if (rounds == 1 || cost < least) {
+      ax = len;
+      least = cost;
+    }
+  }
   const dim3 g(strips, (d.nx + ax - 1) / ax), b(kLanes, ROWS);
   const size_t lds = (size_t)2 * ROWS * kLanes * V * sizeof(float);
   LEX_LAUNCH(KID_ACOUSTIC2, (k_acoustic2<V, MZ, kLanes * ROWS>), g, b, lds, st, d, a, ax);

@@ -114,9 +114,11 @@ def test_acoustic_substep_of_a_blown_up_state(shape, levels):
 
 
 # one and two levels per lane, columns of one wave and of two, full and partial strips of
-# rows, marches of one and of several cells, the last one shorter
+# rows, marches of one and of several cells, the last one shorter; one and several rounds of
+# workgroups, more strips than a round has
 @pytest.mark.parametrize("shape", [(6, 6, 24), (7, 13, 64), (100, 13, 40), (17, 9, 65), (33, 21, 128), (9, 7, 129),
-                                   (20, 9, 256), (181, 147, 71), (300, 60, 33)], ids=str)
+                                   (20, 9, 256), (181, 147, 71), (300, 60, 33), (23, 3200, 6), (19, 1310, 65),
+                                   (40, 530, 130)], ids=str)
 def test_acoustic_pair_is_two_substeps(shape):
     """Two substeps in one launch equal two launches bit for bit; the input's ghosts are not
     periodic images."""
