@@ -790,7 +790,7 @@ __global__ void __launch_bounds__(MAXT) k_acoustic2(Dims d, AcousticArgs a, int 
   }
 }
 
-// Columns of at most two waves; a taller one would leave a workgroup too few rows.
+// Columns of at most three waves; a taller one would leave a workgroup too few rows.
 inline bool acoustic2_ok(const Dims& d) { return d.nz <= 256; }
 
 // ROWS: two levels per lane need 142 to 160 VGPRs, three waves per SIMD, so one workgroup of
@@ -799,11 +799,14 @@ inline bool acoustic2_ok(const Dims& d) { return d.nz <= 256; }
 // taking ax + 3.  One round is best while its strips divide the CUs; us with one round and with
 // this plan, 500x520x130 (131 strips) 2130 and 1082, 1024x1024x32 (171 of 512) 1587 and 869,
 // 300x1600x40 939 and 456, 512x512x100 620 and 540, 240x240x120 (24) 141 and 141.
+// 129 to 192 levels on wide grids: three waves of one level per row instead of two of two levels,
+// the second of which would be part empty; us with two and with three, 150x130x160 97 and 122,
+// 200x200x192 194 and 221, 300x200x129 270 and 247, 256x256x160 296 and 260, 512x300x192 691 and 625.
 template <int V, bool MZ, int ROWS>
 inline void launch_acoustic2_v(const Dims& d, const AcousticArgs& a, hipStream_t st) {
-  constexpr int kLanes = MZ ? 128 : 64;
+  constexpr int kLanes = MZ ? (V == 1 ? 192 : 128) : 64;
   const int strips = (d.ny + ROWS - 3) / (ROWS - 2);
-  const long slots = (long)device_cus() * (V == 1 ? 2 : 1);
+  const long slots = (long)device_cus() * (V == 1 && !MZ ? 2 : 1);
   int ax = d.nx;
   long least = 0;
   for (int rounds = 1; rounds <= 8; ++rounds) {
@@ -814,6 +817,7 @@ inline void launch_acoustic2_v(const Dims& d, const AcousticArgs& a, hipStream_t
       least = cost;
     }
   }
+  if (V == 1 && MZ) ax = std::min(ax, 24);   // of five rows two are halo: neighbours close enough to share them in L2
   const dim3 g(strips, (d.nx + ax - 1) / ax), b(kLanes, ROWS);
   const size_t lds = (size_t)2 * ROWS * kLanes * V * sizeof(float);
   LEX_LAUNCH(KID_ACOUSTIC2, (k_acoustic2<V, MZ, kLanes * ROWS>), g, b, lds, st, d, a, ax);
@@ -823,6 +827,8 @@ inline void launch_acoustic2(const Dims& d, const AcousticArgs& a, hipStream_t s
     launch_acoustic2_v<1, false, 8>(d, a, st);
   else if (d.nz <= 128)
     launch_acoustic2_v<2, false, 12>(d, a, st);
+  else if (d.nz <= 192 && (long)d.nx * d.ny >= 50000)
+    launch_acoustic2_v<1, true, 5>(d, a, st);
   else
     launch_acoustic2_v<2, true, 6>(d, a, st);
 }
