@@ -446,9 +446,9 @@ inline void launch_acoustic(const Dims& d, const AcousticArgs& a, hipStream_t st
 // Bound by memory (the thirteen fields once for two substeps: 72 us at 240x240x120 and
 // 5 TB/s) and by the barrier that holds a CU's waves together.  us per pair against two
 // k_acoustic launches: 40x40x40 9.8 and 19, 96x96x48 19 and 23, 128x128x64 23 and 31,
-// 181x147x70 57 and 64, 192x160x96 65 and 76, 128x128x160 80 and 86, 240x240x120 142 and 198,
-// 256x256x128 152 and 228, 256x256x200 309 and 441, 512x512x64 337 and 438, so every pair of
-// substeps takes it.  With a cell per thread, faces evaluated twice and the levels exchanged
+// 181x147x70 53 and 61, 192x160x96 64 and 73, 240x240x120 141 and 195, 256x256x128 150 and 225,
+// 256x256x200 309 and 441, 512x512x64 300 and 437 (acoustic_pairs has the shapes where two
+// launches win).  With a cell per thread, faces evaluated twice and the levels exchanged
 // through the LDS pipe it took 194 and 194 at 240x240x120 and 256x256x128.  Eight rows of two
 // levels per lane: 166 and 188, sixteen (spills) 172 and 194.
 template <int V>
@@ -792,6 +792,20 @@ __global__ void __launch_bounds__(MAXT) k_acoustic2(Dims d, AcousticArgs a, int 
 
 // Columns of at most three waves; a taller one would leave a workgroup too few rows.
 inline bool acoustic2_ok(const Dims& d) { return d.nz <= 256; }
+
+// Whether a step takes its substeps in pairs.  A pair costs by rows, whatever their levels; two
+// substeps in the caches cost little more than their launches.  us of two substeps and of a pair:
+// shallow and wide 256x256x20 63 and 78, 512x512x16 184 and 280, 512x300x20 109 and 156,
+// 256x256x48 73 and 79, against 128x128x20 26 and 22, 200x200x20 46 and 47, 1024x512x20 445 and
+// 449, 300x200x64 72 and 66, 512x300x48 215 and 178; in part empty waves 96x96x160 43 and 53,
+// 128x128x192 68 and 78, 192x160x144 119 and 145, against 200x200x160 204 and 189.
+inline bool acoustic_pairs(const Dims& d) {
+  const long columns = (long)d.nx * d.ny, cells = columns * d.nz;
+  if (!acoustic2_ok(d)) return false;
+  if (d.nz <= 64) return columns < 40000 || (d.nz > 24 && cells >= 3600000);
+  if (d.nz > 128 && d.nz <= 192) return cells >= 5200000;
+  return true;
+}
 
 // ROWS: two levels per lane need 142 to 160 VGPRs, three waves per SIMD, so one workgroup of
 // twelve waves fills a CU; with one level (87 VGPRs) two workgroups of eight.  The march is the

@@ -486,8 +486,8 @@ int rk3_step(const Dims& d, const O& o, const B& b, float* const* state, char* w
       dts = (float)dts_small;
     }
     float* in[4] = {X0[1], X0[2], X0[3], X0[4]};
-    // the fused path advances two substeps per launch while two remain
-    const bool pairs = (o.solver != 3) && (o.impl == 0) && acoustic2_ok(d);
+    // the fused path advances two substeps per launch while two remain, where that is faster
+    const bool pairs = (o.solver != 3) && (o.impl == 0) && acoustic_pairs(d);
     for (int t = 0; t < nsub;) {
       const int tn = t + ((pairs && t + 1 < nsub) ? 2 : 1);
       float* out[4];

@@ -19,9 +19,10 @@ def _case(nx, ny, nz, passive, seed=3):
 
 
 # marches of 1, 2, 5, 9 and 16 cells with full and partial last tiles, ny mod 4 of 0..3,
-# one, two and three waves per column
+# one, two and three waves per column; substeps in pairs and (the last three) one by one
 @pytest.mark.parametrize("shape,passive", [((8, 9, 16), 0), ((40, 41, 40), 0), ((67, 62, 64), 2), ((97, 91, 70), 1),
-                                           ((157, 160, 130), 2)], ids=str)
+                                           ((157, 160, 130), 2), ((203, 199, 9), 0), ((201, 202, 50), 1),
+                                           ((30, 23, 150), 0)], ids=str)
 def test_stage_tiles_equal_per_operator_kernels(shape, passive):
     """One step with the stage kernel against one kernel per reference routine: the same
     arithmetic up to operation order, a few FP32 ulps of each field (64, as for the other
