@@ -9,8 +9,8 @@
 // cell-per-thread form 77 % busy (29 loads per cell; here 10 for one level, 20 of 8 bytes
 // for two).
 //
-// Contraction is spelled out (fmaf) and otherwise off, in k_acoustic and in both substeps of
-// k_acoustic2, so the results do not depend on which of them computed a cell.
+// Contraction is spelled out (fmaf) and otherwise off, in k_acoustic, in k_acoustic_cells and
+// in both substeps of k_acoustic2, so the results do not depend on which of them computed a cell.
 #pragma once
 #include <algorithm>
 #include "lex_ops.hip"
@@ -325,8 +325,8 @@ __global__ void __launch_bounds__(256) k_acoustic(Dims d, const float* __restric
   }
 }
 
-// The same substep with a thread per cell, which takes every face twice but loads nothing that
-// depends on anything else: for columns of more than two waves.
+// The same substep with a thread per cell, which evaluates every face twice and loads 29 values
+// at once: for columns of more than two waves.
 __global__ void __launch_bounds__(256) k_acoustic_cells(Dims d, const float* __restrict__ rc,
                                                         const float* __restrict__ pi0c, const float* __restrict__ u,
                                                         const float* __restrict__ v, const float* __restrict__ w,

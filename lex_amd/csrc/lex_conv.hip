@@ -571,9 +571,8 @@ constexpr int XR = 24;
 // serve all of a wave's taps.  The two waves of a SIMD hold the larger and the smaller share of
 // pairs.  Neighbouring cells are transposed two at a time, so that LDS takes 4-byte writes.
 // Four waves, one per SIMD (487 VGPRs), that took single taps waited for the tile's loads, read
-// G again for every tap and wrote 2-byte scatters: us per call (22 to 25 of them around the
-// kernel) at 96x96x48, 16->16, 16->32, 32->16 and 32->32 channels, 67, 74, 110 and 127; now 35,
-// 42, 46 and 56.
+// G again for every tap and wrote 2-byte scatters: us of the kernel at 96x96x48, 16->16, 16->32,
+// 32->16 and 32->32 channels, 55, 61, 95 and 112; now 25, 31, 34 and 42.
 // Workgroup b stores its partial sums at part + b * (27 CIN COUT + COUT): the weights' (the two
 // halves added through LDS), then (with_bias) the bias gradient's, which rides along: once a G
 // tile is in LDS, the 512 / COUT threads of each channel row add their consecutive cells of it,

@@ -635,7 +635,7 @@ __device__ __forceinline__ void scalar_tile(const Dims& d, const StageTile& tb, 
 // workgroups of one tile are consecutive, run on one XCD and share the tile's u, v, w
 // lines in its L2.  One launch instead of four (u, v, w, scalars) keeps the chip full where
 // a piece alone would leave it idle, and has one last round instead of four: VALU issue
-// bounds it on large grids (256x256x128, four scalars: 595 us in four launches, 534 in
+// bounds it on large grids (256x256x128, four scalars: 571 us in four launches, 506 in
 // one), the length of a workgroup's march on small ones (40x40x40, two scalars: 132 us per
 // stage in four launches of 16-cell marches, 13 in one of two-cell marches).
 // ---------------------------------------------------------------------------------

@@ -309,8 +309,8 @@ __global__ void __launch_bounds__(kBicgThreads) k_bicg_init(Dims d, const float*
 // sizes solved here stay in the caches and a kernel is one chain of launch, loads, block
 // reduction, arithmetic, block reduction.  So everything a thread reads - its first two
 // cells' operands, the partial sums, the loop state - is requested before the first wait,
-// and each sum is reduced by one kernel only.  64x64x40, us per launch of K1, K2, K3: 6.2, 5.2, 5.8
-// (20.3, 20.7, 20.6 with a wait per array and per cell, 64-bit indices and a pointer table
+// and each sum is reduced by one kernel only.  64x64x40, us per launch of K1, K2, K3: 6.5, 5.5, 5.7
+// (20.5, 21.1, 21.0 with a wait per array and per cell, 64-bit indices and a pointer table
 // in LDS; an empty kernel of this grid takes 2.7).
 constexpr int kBicgAhead = 2;   // cells of a thread whose operands are requested up front
 
