@@ -398,8 +398,9 @@ inline void launch_acoustic_v(const Dims& d, const AcousticArgs& a, hipStream_t 
   // 128x96x96 20.2, 20.9, 19.9, -; 150x130x80 27.0, 25.3, 27.3, -; 192x160x96 43.6, 38.8, -, 40.9;
   // 200x200x80 49.6, 43.2, 40.3, 43.5; 240x240x120 111, 99, -, 97; 256x256x128 129, 115, -, 113.
   const long waves = (long)d.nx * d.ny * chunks;
-  const int ax = V == 1 ? (int)std::min(2L, std::max(1L, (waves + 8192) / 16384))
-                        : (int)std::min(4L, std::max(1L, (waves + 14000) / 16384));
+  const int fill = V == 1 ? (int)std::min(2L, std::max(1L, (waves + 8192) / 16384))
+                          : (int)std::min(4L, std::max(1L, (waves + 14000) / 16384));
+  const int ax = std::max(fill, (d.nx + 65535) / 65536);   // the grid's second dimension holds 2^16
   LEX_LAUNCH(KID_ACOUSTIC, (k_acoustic<V, MZ>), dim3((d.ny + 3) / 4, (d.nx + ax - 1) / ax, chunks), dim3(64, 4, 1), 0, st,
              d, a.rc, a.pi0, a.u, a.v, a.w, a.p, a.ps, a.ru, a.rv, a.rw, a.tr, a.uo, a.vo, a.wo, a.po, a.dts, ax);
 }
@@ -425,8 +426,8 @@ inline void launch_acoustic(const Dims& d, const AcousticArgs& a, hipStream_t st
     launch_acoustic_v<1, false>(d, a, st);
   else if (d.nz <= 128)
     launch_acoustic_v<2, false>(d, a, st);
-  else if (d.nz > 192 && d.nz <= 256 && (cells < 1500000 || cells >= 5000000))
-    launch_acoustic_v<2, true>(d, a, st);
+  else if ((d.nz > 192 && d.nz <= 256 && (cells < 1500000 || cells >= 5000000)) || d.nx >= 65536)
+    launch_acoustic_v<2, true>(d, a, st);   // also where a launch has no place for the cells' x
   else
     launch_acoustic_cells(d, a, st);
 }

@@ -1,6 +1,6 @@
 """CPU oracle: a NumPy restatement of LEX's per-step dynamics (test infrastructure only).
 
-This module is the checker for the HIP path in ``lex_amd``.  Only ``tests/``,
+This module is the oracle for the HIP path in ``lex_amd``.  Only ``tests/``,
 ``__graft_entry__.smoke()`` and the ``cpu_baseline`` leg of ``bench.py`` may import
 it; the product path never calls it.
 

@@ -116,10 +116,10 @@ def test_acoustic_substep_of_a_blown_up_state(shape, levels):
 
 # one and two levels per lane, columns of one wave and of two, full and partial strips of
 # rows, marches of one and of several cells, the last one shorter; one and several rounds of
-# workgroups, more strips than a round has
+# workgroups, more strips than a round has; more cells in x than a launch's second and third dimension
 @pytest.mark.parametrize("shape", [(6, 6, 24), (7, 13, 64), (100, 13, 40), (17, 9, 65), (33, 21, 128), (9, 7, 129),
                                    (20, 9, 256), (181, 147, 71), (300, 60, 33), (23, 3200, 6), (19, 1310, 65),
-                                   (40, 530, 130), (401, 127, 129), (251, 203, 192)], ids=str)
+                                   (40, 530, 130), (401, 127, 129), (251, 203, 192), (65543, 6, 129), (132009, 6, 9)], ids=str)
 def test_acoustic_pair_is_two_substeps(shape):
     """Two substeps in one launch equal two launches bit for bit; the input's ghosts are not
     periodic images."""
